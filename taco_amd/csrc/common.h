@@ -41,6 +41,11 @@ int read_back_i32(const int32_t* src, int n, int32_t* dst, hipStream_t st);
 // Zeroes `bytes` (a multiple of 4) at the 4-byte-aligned p with a kernel on
 // st: unlike hipMemsetAsync, safe inside a HIP graph capture.
 int zero_fill(void* p, size_t bytes, hipStream_t st);
+// pos[0..m] from the non-negative counts[0..m) on st (exclusive prefix sum,
+// pos[m] the sum); *status gets bit 2 on int32 overflow, *total (if given)
+// pos[m].
+int device_counts_to_pos(int32_t m, const int32_t* counts, int32_t* pos,
+                         int32_t* status, hipStream_t st, int32_t* total = nullptr);
 
 // Value types carried by descriptors (csize, in bits).
 enum class VType { F64, F32, BF16, Invalid };

@@ -23,9 +23,6 @@
 
 namespace taco_hip {
 
-int device_counts_to_pos(int32_t m, const int32_t* counts, int32_t* pos,
-                         int32_t* status, hipStream_t st);
-
 namespace {
 
 typedef short v4i16 __attribute__((ext_vector_type(4)));

@@ -1,0 +1,95 @@
+"""SpGEMM rows of more than 64 candidates: every route of the wave-per-row
+kernels (flags, bits, register sorts of 2 to 16 values a lane, hash set;
+sums by column, by staged and by unstaged search), at the edges between them,
+against the oracle: pos and crd bit for bit, and the values too, since every
+column sums separately rounded products in encounter order."""
+import numpy as np
+import pytest
+
+import oracle
+from taco_amd import workloads as W
+from tests import gpu_util as G
+
+pytestmark = pytest.mark.gpu
+
+
+def _csr(rows, n, seed):
+    pos = np.zeros(len(rows) + 1, np.int32)
+    pos[1:] = np.cumsum([len(r) for r in rows])
+    crd = np.concatenate([np.asarray(r, np.int64) for r in rows]).astype(np.int32)
+    vals = W.uniform(len(crd), seed, W.STREAM_VALS)
+    return W.Csr(len(rows), n, pos, crd, vals)
+
+
+def _pick(rng, lo, span, count):
+    """count distinct sorted columns of [lo, lo + span), both ends among them."""
+    inner = rng.choice(span - 2, count - 2, replace=False) + 1 if count > 2 else []
+    return lo + np.sort(np.concatenate([[0], inner, [span - 1]])).astype(np.int64)
+
+
+def _case(span, la, lb, seed, reverse=False):
+    """C rows of la * lb candidates whose columns span exactly `span`; 37
+    rows of C, every B row of a C row from the same window."""
+    rng = np.random.default_rng(seed)
+    m, n = 37, span + 4096
+    brows, arows = [], []
+    for i in range(m):
+        lo = int(rng.integers(0, n - span + 1))
+        arows.append(range(i * la, (i + 1) * la))
+        for _ in range(la):
+            r = _pick(rng, lo, span, min(lb, span))
+            brows.append(r[::-1] if reverse else r)
+    return _csr(arows, m * la, seed), _csr(brows, n, seed + 1)
+
+
+CASES = [
+    # span, A entries, B entries a row
+    ("flags_small", (65, 3, 64)), ("flags_edge", (1024, 5, 70)), ("bits_edge", (1025, 5, 70)),
+    ("bits_mid", (20000, 9, 33)), ("bits_top", (32768, 12, 40)), ("sort_2", (32769, 2, 64)),
+    ("sort_2_65", (40000, 13, 5)), ("sort_4", (40000, 3, 43)), ("sort_4_top", (40000, 4, 64)),
+    ("sort_8", (70000, 257, 1)), ("sort_8_top", (70000, 4, 128)), ("sort_16", (70000, 9, 57)),
+    ("sort_16_top", (70000, 8, 128)), ("hash", (70000, 41, 25)),
+    # distinct columns around the staged-search limit (682) and the slots (1024)
+    ("staged_top", (60000, 11, 62)), ("unstaged", (60000, 11, 63)), ("slots", (50000, 8, 128)),
+    ("over_slots", (300000, 30, 60)), ("long_b", (900, 3, 700)), ("many_a", (1000, 200, 3)),
+]
+
+
+@pytest.mark.parametrize("name,shape", CASES, ids=[c[0] for c in CASES])
+@pytest.mark.parametrize("reverse", [False, True], ids=["sorted", "reversed"])
+def test_mid_rows(name, shape, reverse):
+    A, B = _case(*shape, seed=len(name) * 31 + shape[0], reverse=reverse)
+    print(f"spgemm mid {name} reverse={reverse}", flush=True)
+    pos, crd, vals = G.spgemm(A, B)
+    opos, ocrd = oracle.spgemm_assemble(A, B)
+    assert np.array_equal(pos, opos) and np.array_equal(crd, ocrd)
+    assert np.array_equal(vals, oracle.spgemm_compute(A, B, opos, ocrd))
+
+
+@pytest.mark.parametrize("m", [1, 7, 63, 65, 300])
+def test_mid_rows_among_short_and_empty(m):
+    """Rows of every kind interleaved, at row counts around a workgroup's
+    share."""
+    rng = np.random.default_rng(m)
+    k, n = 500, 3000
+    B = _csr([np.sort(rng.choice(n, int(c), replace=False))
+              for c in rng.choice([0, 1, 5, 40, 90], k)], n, m + 1)
+    A = _csr([np.sort(rng.choice(k, int(c), replace=False))
+              for c in rng.choice([0, 1, 3, 10, 70], m)], k, m + 2)
+    pos, crd, vals = G.spgemm(A, B)
+    opos, ocrd = oracle.spgemm_assemble(A, B)
+    assert np.array_equal(pos, opos) and np.array_equal(crd, ocrd)
+    assert np.array_equal(vals, oracle.spgemm_compute(A, B, opos, ocrd))
+
+
+def test_subnormal_sums():
+    """Products and sums of multiples of 2^-1074 are exact: sums in LDS must
+    not flush them.  Compared as integers (a host in flush-to-zero mode would
+    compare the floats as equal)."""
+    k = np.arange(1, 211, dtype=np.int64)
+    B = W.Csr(70, 3, np.arange(0, 211, 3, dtype=np.int32), np.tile(np.arange(3, dtype=np.int32), 70),
+              k.view(np.float64))
+    A = W.Csr(1, 70, np.array([0, 70], np.int32), np.arange(70, dtype=np.int32), np.ones(70))
+    _, crd, vals = G.spgemm(A, B)
+    assert crd.tolist() == [0, 1, 2]
+    assert vals.view(np.int64).tolist() == k.reshape(70, 3).sum(0).tolist()
