@@ -212,8 +212,9 @@ __global__ __launch_bounds__(256) void k_spgemm_numeric_short(
 // consecutive rows, reads which of them are its own kind with one coalesced
 // load and deals them to its four waves in row order.  A list needs an
 // atomic per row on one counter: with 100,003 rows to list the short-row
-// kernels took 1.07 ms each, without the list 16 and 26 us.  Neighbouring rows also stay together, so
-// rows of a banded product find their B rows in L1 and L2.
+// kernels took 1.07 ms each, without the list 16 and 26 us.  Neighbouring
+// rows also stay together, so rows of a banded product find their B rows in
+// L1 and L2.
 
 // Rows a workgroup takes: 16384 workgroups or more (64 a CU) as soon as the
 // rows allow, so that the last ones level out (100,003 banded rows, 4

@@ -158,32 +158,6 @@ __global__ __launch_bounds__(256) void k_spmm_nnz_split(
   }
 }
 
-// Merge-path split (see wave_merge_search) for a team of G lanes.
-template <int G>
-__device__ __forceinline__ int64_t group_merge_search(const int32_t* pos,
-                                                      int64_t m, int64_t nnz,
-                                                      int64_t d) {
-  int64_t lo = d - nnz > 0 ? d - nnz : 0;
-  int64_t hi = d < m ? d : m;
-  const int lane = (int)__lane_id() & (G - 1);
-  const int base = (int)__lane_id() & ~(G - 1);
-  while (lo < hi) {
-    const int64_t step = (hi - lo + G - 1) / G;
-    const int64_t p = lo + (int64_t)lane * step;
-    bool pred = false;
-    if (p < hi) pred = (int64_t)pos[p + 1] <= d - p - 1;
-    uint64_t mask = __ballot(pred) >> base;
-    if (G < 64) mask &= ((1ull << G) - 1);
-    const int c = __popcll(mask);
-    const int64_t nlo = c == 0 ? lo : lo + (int64_t)(c - 1) * step + 1;
-    int64_t nhi = lo + (int64_t)c * step;
-    if (nhi > hi) nhi = hi;
-    lo = nlo;
-    hi = nhi;
-  }
-  return lo;
-}
-
 // Value of lane `idx` of this lane's team of G lanes (idx uniform across
 // the team).  A whole-wave team reads it with v_readlane into a scalar.
 template <int G, typename T>
@@ -202,128 +176,322 @@ __device__ __forceinline__ T team_bcast(T v, int idx) {
   }
 }
 
-template <typename TA, typename TC, int G, int CPL>
+// W adjacent values, aligned as one of them.
+template <typename T, int W>
+struct Adjacent;
+#define TH_ADJACENT(T, W)                                                        \
+  template <>                                                                    \
+  struct Adjacent<T, W> {                                                        \
+    typedef T vec __attribute__((ext_vector_type(W), aligned(sizeof(T))));       \
+  };
+TH_ADJACENT(double, 1) TH_ADJACENT(double, 2) TH_ADJACENT(double, 4)
+TH_ADJACENT(float, 1) TH_ADJACENT(float, 2) TH_ADJACENT(float, 4)
+TH_ADJACENT(uint16_t, 1) TH_ADJACENT(uint16_t, 2) TH_ADJACENT(uint16_t, 4)
+#undef TH_ADJACENT
+template <int W>
+__device__ __forceinline__ void load_wide(const double* p, double (&out)[W]) {
+  const typename Adjacent<double, W>::vec v = *(const typename Adjacent<double, W>::vec*)p;
+#pragma unroll
+  for (int c = 0; c < W; ++c) out[c] = v[c];
+}
+template <int W>
+__device__ __forceinline__ void load_wide(const float* p, float (&out)[W]) {
+  const typename Adjacent<float, W>::vec v = *(const typename Adjacent<float, W>::vec*)p;
+#pragma unroll
+  for (int c = 0; c < W; ++c) out[c] = v[c];
+}
+template <int W>
+__device__ __forceinline__ void load_wide(const bf16_t* p, float (&out)[W]) {
+  const typename Adjacent<uint16_t, W>::vec v = *(const typename Adjacent<uint16_t, W>::vec*)p;
+#pragma unroll
+  for (int c = 0; c < W; ++c) out[c] = widen(bf16_t{v[c]});
+}
+
+// One wave per team.  L = ceil(K / CPL) lanes cover the K columns, each
+// owning CPL adjacent ones: its first column is kl * CPL, or K - CPL where
+// that would pass the end, so that every lane loads CPL columns of a B row in
+// one go (16 bytes for four f32 or two f64 columns); the last two lanes may
+// overlap and then hold the same sums.  The wave's S = 64 / L groups of L
+// lanes take consecutive entries, so that one load instruction gathers S B
+// rows; a finished row's sums are added across the groups.  Wide loads and
+// full waves are what counts where B's rows come from the caches: the L1's
+// data path works by the lane, whether it is of use or not.  (ONE: a wave to
+// a B row, whose address and value then sit in scalar registers.)
+//
+// Entries are taken in blocks, U steps of S of them (S * U <= 64), whatever
+// rows they belong to: a block's B rows are gathered together, then added step by
+// step with the row ends in between.  The next chunk's columns and values
+// load while the current one is worked on, and 64 row ends are held in the
+// lanes, so no step waits for a chain of dependent loads; the walk itself is
+// the same for the whole wave and runs on the scalar unit.
+//
+// 400,009 banded rows of 24 entries, K = 33, f32: 294 us with one row at a
+// time (pos, then its entries, then B rows, each waited for; a row's last
+// entries one by one; one B row to a load), 179 us now: the L1 fetches 1.7
+// lines of B from L2 for an entry, 1.9 GB at the 18 TB/s that L2 delivers
+// being 104 us of it.  1M-row power-law matrix, K = 64, f64: 1295 -> 1210 us,
+// 64 M lines of B, at the 53 G random lines a second that the card delivers.
+template <typename TA, typename TC, int CPL, int U, bool ONE>
 __global__ __launch_bounds__(256) void k_spmm_merge(
     int32_t m, int64_t nnz, int32_t K, int32_t items_per_team,
     const int32_t* __restrict__ pos, const int32_t* __restrict__ crd,
     const TA* __restrict__ vals, const TA* __restrict__ B,
     TC* __restrict__ C, int64_t nteams, int32_t* __restrict__ carry_row,
     TC* __restrict__ carry_val) {
-  const int lane = threadIdx.x & (G - 1);
-  const int64_t team = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / G;
-  // Whole teams only: the grid is sized so a team is either fully in range
-  // or fully out, and ballots inside the search see complete teams.
+  typedef typename Adjacent<TC, CPL>::vec Out;
+  const int lane = threadIdx.x % kWave;
+  const int L = (K + CPL - 1) / CPL;
+  const int S = ONE ? 1 : kWave / L < kWave / U ? kWave / L : kWave / U;
+  const int chunk = kWave / (S * U) * (S * U);
+  const int sub = ONE ? 0 : lane / L, kl = ONE ? lane : lane % L;
+  const bool owns = sub < S && kl < L;  // lanes left over repeat others' loads
+  const int64_t team = (int64_t)blockIdx.x * (256 / kWave) +
+                       __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
   if (team >= nteams) return;
   const int64_t total = (int64_t)m + nnz;
-  int64_t d = team * items_per_team;
-  const int64_t dend = d + items_per_team < total ? d + items_per_team : total;
-  int64_t r = group_merge_search<G>(pos, m, nnz, d);
-  int64_t z = d - r;
+  const int64_t d0 = team * items_per_team;
+  int32_t left = (int32_t)(total - d0 < items_per_team ? total - d0 : items_per_team);
+  int32_t r = __builtin_amdgcn_readfirstlane((int)wave_merge_search(pos, m, nnz, d0));
+  int32_t z = (int32_t)(d0 - r);
+  // kStrided: a lane's columns are lane, lane + 64, ... instead, those past
+  // the end repeating column K - 1.
+  constexpr bool kStrided = ONE && sizeof(TC) == 8;
+  const int32_t k0 = kStrided ? 0 : kl * CPL < K - CPL ? kl * CPL : K - CPL;
+  const bool stores = sub == 0 && owns;
+  int32_t ks[CPL];
+#pragma unroll
+  for (int c = 0; c < CPL; ++c) ks[c] = lane + c * kWave < K ? lane + c * kWave : K - 1;
+  const auto store_row = [&](TC* row, Out sum, bool stream) {
+    if constexpr (kStrided) {
+#pragma unroll
+      for (int c = 0; c < CPL; ++c) {
+        if (lane + c * kWave >= K) continue;
+        if (stream)
+          __builtin_nontemporal_store((TC)sum[c], row + lane + c * kWave);
+        else
+          row[lane + c * kWave] = sum[c];
+      }
+    } else if (stores) {
+      if (stream)
+        __builtin_nontemporal_store(sum, (Out*)(row + k0));
+      else
+        *(Out*)(row + k0) = sum;
+    }
+  };
   TC acc[CPL];
 #pragma unroll
   for (int c = 0; c < CPL; ++c) acc[c] = 0;
-  bool partial = false;  // acc holds entries of row r
-  while (d < dend) {
-    const int64_t rend = pos[r + 1];  // r < m while items remain
-    int64_t zstop = z + (dend - d);
-    if (zstop > rend) zstop = rend;
-    const int64_t take = zstop - z;
-    if (take > 0) partial = true;
-    // The team loads up to G consecutive entries at once (one per lane,
-    // coalesced) and broadcasts them one by one; 8 B-row gathers in flight.
-    for (int64_t zc = z; zc < zstop; zc += G) {
-      const int cnt = (int)(zstop - zc < G ? zstop - zc : G);
-      const int32_t jl = lane < cnt ? stream_load(crd + zc + lane) : 0;
-      const TC al = lane < cnt ? widen(stream_load(vals + zc + lane)) : TC(0);
-      int u = 0;
-      for (; u + 8 <= cnt; u += 8) {
-        int32_t j[8];
-        TC a[8];
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-          j[q] = team_bcast<G>(jl, u + q);
-          a[q] = team_bcast<G>(al, u + q);
-        }
-        TC b[8][CPL];
-#pragma unroll
-        for (int q = 0; q < 8; ++q)
-#pragma unroll
-          for (int c = 0; c < CPL; ++c) {
-            const int k = lane + c * G;
-            b[q][c] = k < K ? widen(B[(int64_t)j[q] * K + k]) : TC(0);
-          }
-#pragma unroll
-        for (int q = 0; q < 8; ++q)
-#pragma unroll
-          for (int c = 0; c < CPL; ++c) acc[c] += a[q] * b[q][c];
-      }
-      for (; u < cnt; ++u) {
-        const int32_t j = team_bcast<G>(jl, u);
-        const TC a = team_bcast<G>(al, u);
+  // The row's sums, added across the lane groups, in group 0.
+  const auto row_sum = [&]() {
+    if constexpr (!ONE) {
+      for (int g = S > 8 ? 8 : S > 4 ? 4 : S > 2 ? 2 : S > 1 ? 1 : 0; g > 0; g >>= 1) {
+        const bool have = sub + g < S;
+        const int from = have ? lane + g * L : lane;
 #pragma unroll
         for (int c = 0; c < CPL; ++c) {
-          const int k = lane + c * G;
-          if (k < K) acc[c] += a * widen(B[(int64_t)j * K + k]);
+          const TC v = __shfl(acc[c], from, kWave);
+          acc[c] = have ? acc[c] + v : acc[c];
         }
       }
     }
-    z = zstop;
-    d += take;
-    if (d < dend && z == rend) {
-      // Row end item: row r completes in this team (its earlier entries, if
-      // any, arrive through the carries of preceding teams).
-#pragma unroll
-      for (int c = 0; c < CPL; ++c) {
-        const int k = lane + c * G;
-        // non-temporal: C is written once, B rows keep the caches
-        if (k < K) __builtin_nontemporal_store(acc[c], C + r * K + k);
-        acc[c] = 0;
-      }
-      partial = false;
-      ++r;
-      ++d;
-    }
-  }
-  const bool has_carry = partial && r < m;
-  if (lane == 0) carry_row[team] = has_carry ? (int32_t)r : -1;
-  if (has_carry) {
+    Out sum;
 #pragma unroll
     for (int c = 0; c < CPL; ++c) {
-      const int k = lane + c * G;
-      if (k < K) carry_val[team * K + k] = acc[c];
+      sum[c] = acc[c];
+      acc[c] = 0;
+    }
+    return sum;
+  };
+  // Ends of the rows first .. first + 63; row m's never comes.
+  const auto row_ends = [&](int32_t first) {
+    const int64_t q = (int64_t)first + 1 + lane;
+    return q <= m ? pos[q] : INT_MAX;
+  };
+  int at = 0;
+  int32_t ends = row_ends(r);
+  int32_t rend = __builtin_amdgcn_readlane(ends, 0);
+  int32_t zrow = z;  // the team's first entry of row r
+  // Entries past nnz > 0 are loaded as the last one and never added.
+  const auto entry = [&](int32_t first) {
+    const int64_t q = (int64_t)first + lane;
+    return q < nnz ? q : nnz - 1;
+  };
+  int32_t zc = z;
+  int32_t jn = stream_load(crd + entry(zc));
+  TA an = stream_load(vals + entry(zc));
+  while (left > 0) {
+    const int32_t jl = jn;
+    const TC al = widen(an);
+    zc = zc < INT_MAX - kWave ? zc + chunk : zc;
+    jn = stream_load(crd + entry(zc));
+    an = stream_load(vals + entry(zc));
+    for (int e0 = 0; e0 < chunk && left > 0; e0 += S * U) {
+      TC a[U], b[U][CPL];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        int32_t j;
+        if constexpr (ONE) {
+          j = team_bcast<kWave>(jl, e0 + u);
+          a[u] = team_bcast<kWave>(al, e0 + u);
+        } else {
+          j = __shfl(jl, e0 + u * S + sub, kWave);
+          a[u] = __shfl(al, e0 + u * S + sub, kWave);
+        }
+        if constexpr (kStrided) {
+#pragma unroll
+          for (int c = 0; c < CPL; ++c) b[u][c] = widen(B[(int64_t)j * K + ks[c]]);
+        } else {
+          load_wide<CPL>(B + (int64_t)j * K + k0, b[u]);
+        }
+      }
+      if (left >= S * U && rend - z >= S * U) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int c = 0; c < CPL; ++c) acc[c] += a[u] * b[u][c];
+        z += S * U;
+        left -= S * U;
+        continue;
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        int done = 0;  // entries of this step already added
+        do {
+          while (left > 0 && z == rend) {
+            // Row end item: row r completes in this team (its earlier
+            // entries, if any, arrive through the carries of preceding teams).
+            const Out sum = row_sum();
+            // non-temporal: C is written once, B rows keep the caches
+            store_row(C + (int64_t)r * K, sum, true);
+            ++r;
+            --left;
+            zrow = z;
+            if (++at == kWave) {
+              at = 0;
+              ends = row_ends(r);
+            }
+            rend = __builtin_amdgcn_readlane(ends, at);
+          }
+          int take = S - done < rend - z ? S - done : rend - z;
+          take = take < left ? take : left;
+          // Only the entries' own lanes add: a B row outside may hold
+          // infinities or NaN.
+          if (ONE ? take > 0 : sub >= done && sub < done + take) {
+#pragma unroll
+            for (int c = 0; c < CPL; ++c) acc[c] += a[u] * b[u][c];
+          }
+          z += take;
+          left -= take;
+          done += take;
+        } while (left > 0 && done < S);
+      }
+    }
+  }
+  const bool has_carry = z > zrow && r < m;
+  if (lane == 0) carry_row[team] = has_carry ? r : -1;
+  if (has_carry) {
+    const Out sum = row_sum();
+    store_row(carry_val + team * K, sum, false);
+  }
+}
+
+// A wave per carry slot; the first slot of each run of equal rows adds the
+// run.  The rows of 63 slots and the first carry load at once, then C's row:
+// a wave waits for memory twice, which is what this kernel's time is made
+// of.  Runs of up to kFixupOwn slots are added by that wave in team order;
+// longer ones (a row of 1e5 entries leaves some 400) are cut into 4
+// consecutive pieces, one for each wave of the workgroup, whose sums are
+// then added in order: the order is fixed, so results do not change from
+// run to run.  Walking run and carries one after another in one wave, the
+// longest row of a 1M-row power-law matrix at K = 64, f64, kept this kernel
+// busy for 115 us (now 31).
+constexpr int kFixupWaves = 4;
+constexpr int kFixupOwn = 16;
+template <typename TC>
+__device__ __forceinline__ TC add_carries(const TC* __restrict__ carry_val, int64_t q, int64_t e,
+                                          int32_t K, int32_t k, TC s) {
+  for (; q + 16 <= e; q += 16) {
+    TC v[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) v[u] = carry_val[(q + u) * K + k];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) s += v[u];
+  }
+  for (; q < e; ++q) s += carry_val[q * K + k];
+  return s;
+}
+template <typename TC>
+__global__ __launch_bounds__(kFixupWaves * kWave) void k_spmm_merge_fixup(
+    int64_t nteams, int32_t K, const int32_t* __restrict__ carry_row,
+    const TC* __restrict__ carry_val, TC* __restrict__ C) {
+  __shared__ int32_t s_len[kFixupWaves];
+  __shared__ TC s_sum[kFixupWaves][kWave];
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+  const int lane = threadIdx.x % kWave;
+  const int64_t t0 = (int64_t)blockIdx.x * kFixupWaves;
+  const int64_t t = t0 + wave;
+  // Lane l holds the row of slot t - 1 + l; -2 outside the slots.
+  const int64_t q = t - 1 + lane;
+  const int32_t row = q >= 0 && q < nteams ? carry_row[q] : -2;
+  const TC first = t < nteams && lane < K ? carry_val[t * K + lane] : TC(0);
+  const int32_t before = __builtin_amdgcn_readlane(row, 0);
+  const int32_t r = __builtin_amdgcn_readlane(row, 1);
+  int64_t e = t;  // the run is t .. e - 1
+  if (r >= 0 && before != r) {
+    uint64_t other = __ballot(row != r) >> 1;  // bit i: slot t + i is of another row
+    if (other) {
+      e = t + __ffsll((unsigned long long)other) - 1;
+    } else {
+      for (e = t + kWave - 1;; e += kWave) {
+        const int64_t p = e + lane;
+        other = __ballot(p >= nteams || carry_row[p < nteams ? p : t] != r);
+        if (other) {
+          e += __ffsll((unsigned long long)other) - 1;
+          break;
+        }
+      }
+    }
+    if (e - t <= kFixupOwn)
+      for (int32_t k = lane; k < K; k += kWave) {
+        const TC s = k == lane ? first : carry_val[t * K + k];
+        C[(int64_t)r * K + k] += add_carries(carry_val, t + 1, e, K, k, s);
+      }
+  }
+  // At most INT32_MAX teams.
+  if (lane == 0) s_len[wave] = (int32_t)(e - t);
+  __syncthreads();
+  for (int w = 0; w < kFixupWaves; ++w) {
+    const int32_t len = s_len[w];  // the same for the whole workgroup
+    if (len <= kFixupOwn) continue;
+    const int64_t q0 = t0 + w, q1 = q0 + len;
+    const int64_t piece = (len + kFixupWaves - 1) / kFixupWaves;
+    const int64_t a = q0 + wave * piece < q1 ? q0 + wave * piece : q1;
+    const int64_t b = a + piece < q1 ? a + piece : q1;
+    for (int32_t kb = 0; kb < K; kb += kWave) {
+      const int32_t k = kb + lane;
+      s_sum[wave][lane] = k < K ? add_carries(carry_val, a, b, K, k, TC(0)) : TC(0);
+      __syncthreads();
+      if (wave == w && k < K) {
+        TC s = 0;
+        for (int v = 0; v < kFixupWaves; ++v) s += s_sum[v][lane];
+        C[(int64_t)r * K + k] += s;
+      }
+      __syncthreads();
     }
   }
 }
 
-// One 64-lane wave per carry slot; the first slot of each run of equal rows
-// adds the whole run, in team order.
+// Adjacent columns a lane of the merge kernel owns: 16 bytes of f32 or f64
+// (one column below that width), except f64 rows of 33 to 64 columns, where
+// a wave to a B row is faster (1M-row power-law matrix, K = 64: 1210 us
+// against 1245 with two columns a lane).  Wider f64 rows take strided
+// columns (kStrided: 326,797 uniform rows of 30, K = 102: 1272 us against
+// 1307 with adjacent ones; 200,000 banded rows, K = 128: 406 against 430).
 template <typename TC>
-__global__ __launch_bounds__(256) void k_spmm_merge_fixup(
-    int64_t nteams, int32_t K, const int32_t* __restrict__ carry_row,
-    const TC* __restrict__ carry_val, TC* __restrict__ C) {
-  const int64_t t = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave;
-  const int lane = threadIdx.x % kWave;
-  if (t >= nteams) return;
-  const int32_t r = carry_row[t];
-  if (r < 0) return;
-  if (t > 0 && carry_row[t - 1] == r) return;
-  int64_t e = t + 1;
-  while (e < nteams && carry_row[e] == r) ++e;
-  for (int32_t k = lane; k < K; k += kWave) {
-    TC s = carry_val[t * K + k];
-    int64_t q = t + 1;
-    // Loads 8 carries ahead, adds them in team order (long rows have
-    // hundreds of carries; the order of the sum stays fixed).
-    for (; q + 8 <= e; q += 8) {
-      TC v[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = carry_val[(q + u) * K + k];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) s += v[u];
-    }
-    for (; q < e; ++q) s += carry_val[q * K + k];
-    C[(int64_t)r * K + k] += s;
-  }
+int merge_cols(int32_t K) {
+  const int wide = 16 / (int)sizeof(TC);
+  if (sizeof(TC) == 8 && K > 32 && K <= 64) return 1;
+  return K < wide ? 1 : K <= 64 * wide ? wide : 4;
 }
 
 template <typename TA, typename TC>
@@ -389,6 +557,7 @@ int run_spmm(const CsrView& a, int32_t K, const TA* B, TC* C,
     return fail("spmm: no kernel for G=%d CPL=%d", G, CPL);
   }
   if (algo == TACO_HIP_MERGE_PATH) {
+    if (a.nnz == 0) return zero_fill(C, sizeof(TC) * (size_t)a.m * K, st);
     int ipt = s.items_per_thread > 0 ? s.items_per_thread : 256;
     const int64_t total = (int64_t)a.m + a.nnz;
     const int64_t nteams = (total + ipt - 1) / ipt;
@@ -397,21 +566,23 @@ int run_spmm(const CsrView& a, int32_t K, const TA* B, TC* C,
     if (!ws) return 1;
     int32_t* crow = (int32_t*)ws;
     TC* cval = (TC*)((char*)ws + row_bytes);
-    unsigned grid = (unsigned)((nteams + teams_per_block - 1) / teams_per_block);
-    bool launched = false;
-#define TH_X(g, c)                                                          \
-  if (!launched && G == g && CPL == c) {                                    \
-    k_spmm_merge<TA, TC, g, c><<<grid, bs, 0, st>>>(                        \
+    const int cols = merge_cols<TC>(K);
+    const bool one = (K + cols - 1) / cols > 32;
+    unsigned grid = (unsigned)((nteams * kWave + bs - 1) / bs);
+    // Narrow rows: 16 groups of 4 lanes, 4 steps each.
+    const int steps = (K + cols - 1) / cols <= 4 ? 4 : 8;
+#define TH_MERGE(c, u, o)                                                   \
+  if (cols == c && steps == u && one == o)                                  \
+    k_spmm_merge<TA, TC, c, u, o><<<grid, bs, 0, st>>>(                     \
         a.m, a.nnz, K, ipt, a.pos, a.crd, (const TA*)a.vals, B, C, nteams,  \
-        crow, cval);                                                        \
-    launched = true;                                                        \
-  }
-    TH_SHAPES(TH_X)
-#undef TH_X
-    TH_REQUIRE(launched, "spmm: no kernel for G=%d CPL=%d", G, CPL);
+        crow, cval);
+    TH_MERGE(1, 4, false) TH_MERGE(1, 8, false) TH_MERGE(1, 8, true)
+    TH_MERGE(2, 4, false) TH_MERGE(2, 8, false) TH_MERGE(2, 8, true)
+    TH_MERGE(4, 4, false) TH_MERGE(4, 8, false) TH_MERGE(4, 8, true)
+#undef TH_MERGE
     TH_LAUNCH_CHECK("k_spmm_merge");
-    unsigned g2 = (unsigned)((nteams * kWave + 255) / 256);
-    k_spmm_merge_fixup<TC><<<g2, 256, 0, st>>>(nteams, K, crow, cval, C);
+    unsigned g2 = (unsigned)((nteams + kFixupWaves - 1) / kFixupWaves);
+    k_spmm_merge_fixup<TC><<<g2, kFixupWaves * kWave, 0, st>>>(nteams, K, crow, cval, C);
     return 0;
   }
 #undef TH_SHAPES
