@@ -287,25 +287,29 @@ __global__ __launch_bounds__(256) void k_spmv_merge_fixup(
 
 // The merge path's form for few entries (at most kSmallEntries): one launch,
 // no search and no carries.  G lanes take a row; a row of more than
-// kSmallOwn entries a lane is left to the workgroup, whose 256 threads add
-// it up together afterwards.  Sums are taken in a fixed order, without
-// atomics, like the merge path's.
+// kSmallOwn entries a lane is left to the workgroup, whose threads add it up
+// together afterwards.  Sums are taken in a fixed order, without atomics,
+// like the merge path's.
 //
 // Such calls cost launches and chains of dependent loads, not bandwidth: a
 // merge-path call launches twice (3.5 us each back to back) and searches its
-// tile's corners before it loads an entry.  1000 rows of 10, f64: 7.7 -> 3.8 us.
-// The line lies where one row holding all entries (512 a thread, 16 in
-// flight) would take about twice the merge path's time.
-constexpr int64_t kSmallEntries = 1 << 17;
+// tile's corners before it loads an entry.  1000 rows of 10, f64: 7.7 -> 3.8
+// us; 8192 rows of 8: 8.8 -> 3.8.  The line lies where rows that one
+// workgroup has to add up still cost about what the merge path does: half of
+// 65,536 entries in one row take 12.7 us against 10.6, all of them 19.6
+// against 11.3 (131,072: 21 and 37 against 13 and 16).  1024 threads: with
+// 256 those rows took 27 and 49 us at 131,072.
+constexpr int64_t kSmallEntries = 1 << 16;
 constexpr int kSmallOwn = 16;
+constexpr int kSmallThreads = 1024;
 template <typename T, int G>
-__global__ __launch_bounds__(256) void k_spmv_small(
+__global__ __launch_bounds__(kSmallThreads) void k_spmv_small(
     int32_t m, const int32_t* __restrict__ pos, const int32_t* __restrict__ crd,
     const T* __restrict__ vals, const T* __restrict__ x, T* __restrict__ y) {
-  constexpr int kRows = 256 / G;
+  constexpr int kRows = kSmallThreads / G;
   constexpr int kAhead = 4, kLongAhead = 16;
   __shared__ int32_t s_long[kRows];
-  __shared__ T s_sum[256 / kWave];
+  __shared__ T s_sum[kSmallThreads / kWave];
   __shared__ int s_count;
   const int tid = threadIdx.x, sub = tid % G, slot = tid / G;
   const int64_t i = (int64_t)blockIdx.x * kRows + slot;
@@ -337,24 +341,24 @@ __global__ __launch_bounds__(256) void k_spmv_small(
     const int64_t row = (int64_t)blockIdx.x * kRows + s_long[k];
     const int32_t q0 = pos[row], q1 = pos[row + 1];
     T s = 0;
-    for (int32_t p = q0 + tid; p < q1; p += kLongAhead * 256) {
+    for (int32_t p = q0 + tid; p < q1; p += kLongAhead * kSmallThreads) {
       T v[kLongAhead], xv[kLongAhead];
 #pragma unroll
       for (int u = 0; u < kLongAhead; ++u) {
-        const int32_t q = p + u * 256 < q1 ? p + u * 256 : p;
+        const int32_t q = p + u * kSmallThreads < q1 ? p + u * kSmallThreads : p;
         v[u] = vals[q];
         xv[u] = x[crd[q]];
       }
 #pragma unroll
       for (int u = 0; u < kLongAhead; ++u)
-        if (p + u * 256 < q1) s += v[u] * xv[u];
+        if (p + u * kSmallThreads < q1) s += v[u] * xv[u];
     }
     s = wave_sum(s);
     if (tid % kWave == 0) s_sum[tid / kWave] = s;
     __syncthreads();
     if (tid == 0) {
       T all = 0;
-      for (int w = 0; w < 256 / kWave; ++w) all += s_sum[w];
+      for (int w = 0; w < kSmallThreads / kWave; ++w) all += s_sum[w];
       y[row] = all;
     }
     __syncthreads();
@@ -366,10 +370,10 @@ template <typename T>
 void launch_spmv_small(const CsrView& a, const T* x, T* y, hipStream_t st) {
   int g = 2;
   while (g < 64 && (int64_t)g * 3 * a.m < a.nnz) g <<= 1;
-  const unsigned grid = (unsigned)(((int64_t)a.m * g + 255) / 256);
+  const unsigned grid = (unsigned)(((int64_t)a.m * g + kSmallThreads - 1) / kSmallThreads);
 #define TH_SMALL(G)                                                            \
   case G:                                                                      \
-    k_spmv_small<T, G><<<grid, 256, 0, st>>>(a.m, a.pos, a.crd,                \
+    k_spmv_small<T, G><<<grid, kSmallThreads, 0, st>>>(a.m, a.pos, a.crd,      \
                                              (const T*)a.vals, x, y);          \
     break;
   switch (g) {
@@ -442,7 +446,7 @@ int run_spmv(const CsrView& a, const T* x, T* y, const taco_hip_schedule& s,
                "spmv: MERGE_PATH uses 256-thread workgroups");
     TH_REQUIRE(k == 2 || k == 4 || k == 6 || k == 8 || k == 12 || k == 16,
                "spmv: items_per_thread %d unsupported for MERGE_PATH", k);
-    if (a.nnz <= kSmallEntries && (int64_t)a.m <= 8 * kSmallEntries) {
+    if (a.nnz <= kSmallEntries && (int64_t)a.m <= 16 * kSmallEntries) {
       launch_spmv_small<T>(a, x, y, st);
       return 0;
     }

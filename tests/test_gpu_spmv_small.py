@@ -10,7 +10,7 @@ from taco_amd import workloads as W
 from tests import gpu_util as G
 
 pytestmark = pytest.mark.gpu
-LIMIT = 1 << 17
+LIMIT = 1 << 16
 TOL = {"f64": 1e-12, "f32": 1e-5}
 
 
