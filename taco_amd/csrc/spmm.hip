@@ -158,21 +158,16 @@ __global__ __launch_bounds__(256) void k_spmm_nnz_split(
   }
 }
 
-// Value of lane `idx` of this lane's team of G lanes (idx uniform across
-// the team).  A whole-wave team reads it with v_readlane into a scalar.
-template <int G, typename T>
-__device__ __forceinline__ T team_bcast(T v, int idx) {
-  if constexpr (G == 64) {
-    if constexpr (sizeof(T) == 8) {
-      const uint64_t b = __builtin_bit_cast(uint64_t, v);
-      const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, idx);
-      const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), idx);
-      return __builtin_bit_cast(T, ((uint64_t)hi << 32) | lo);
-    } else {
-      return __builtin_bit_cast(T, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), idx));
-    }
+// Value of lane `idx` (wave-uniform), in a scalar register.
+template <typename T>
+__device__ __forceinline__ T wave_bcast(T v, int idx) {
+  if constexpr (sizeof(T) == 8) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, idx);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), idx);
+    return __builtin_bit_cast(T, ((uint64_t)hi << 32) | lo);
   } else {
-    return __shfl(v, idx, G);
+    return __builtin_bit_cast(T, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), idx));
   }
 }
 
@@ -331,8 +326,8 @@ __global__ __launch_bounds__(256) void k_spmm_merge(
       for (int u = 0; u < U; ++u) {
         int32_t j;
         if constexpr (ONE) {
-          j = team_bcast<kWave>(jl, e0 + u);
-          a[u] = team_bcast<kWave>(al, e0 + u);
+          j = wave_bcast(jl, e0 + u);
+          a[u] = wave_bcast(al, e0 + u);
         } else {
           j = __shfl(jl, e0 + u * S + sub, kWave);
           a[u] = __shfl(al, e0 + u * S + sub, kWave);
