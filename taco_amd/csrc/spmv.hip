@@ -311,39 +311,91 @@ __global__ __launch_bounds__(256) void k_spmv_merge_fixup(
   }
 }
 
-// The merge path's form for few entries (at most kSmallEntries): one launch,
-// no search and no carries.  G lanes take a row; a row of more than
-// kSmallOwn entries a lane is left to the workgroup, whose threads add it up
-// together afterwards.  Sums are taken in a fixed order, without atomics,
-// like the merge path's.
+// The merge path's form for few entries (small_spmv): one launch, no search
+// and no carries.  G lanes take a row; rows of more than kSmallOwn entries a
+// lane are left for the workgroup's teams of 16 lanes (up to kSmallTeamRow
+// entries), its waves (up to kSmallWaveRow) or all its threads, so that many
+// of them are summed side by side.  Sums are taken in a fixed order, without
+// atomics, like the merge path's.
 //
 // Such calls cost launches and chains of dependent loads, not bandwidth: a
 // merge-path call launches twice (3.5 us each back to back) and searches its
-// tile's corners before it loads an entry.  1000 rows of 10, f64: 7.7 -> 3.8
-// us; 8192 rows of 8: 8.8 -> 3.8.  The line lies where rows that one
-// workgroup has to add up still cost about what the merge path does: half of
-// 65,536 entries in one row take 12.7 us against 10.6, all of them 19.6
-// against 11.3 (131,072: 21 and 37 against 13 and 16).  1024 threads: with
-// 256 those rows took 27 and 49 us at 131,072.
-constexpr int64_t kSmallEntries = 1 << 16;
+// tile's corners before it loads an entry.
+//
+// Neighbouring rows go to different workgroups (row i to workgroup i %
+// gridDim.x): long rows that lie together, as the border or a dense block of
+// an operator, are spread over the CUs, of which each gathers one line of x
+// a cycle at most.  The number of workgroups is odd, so that long rows at a
+// power of two's distance are spread as well.
 constexpr int kSmallOwn = 16;
 constexpr int kSmallThreads = 1024;
+constexpr int kSmallAhead = 16;
+constexpr int kSmallTeam = 16;
+constexpr int32_t kSmallTeamRow = kSmallTeam * kSmallAhead;
+constexpr int32_t kSmallWaveRow = 2 * kWave * kSmallAhead;
+// Workgroups, rows allowing.
+constexpr int kSmallSpread = 32;
+
+// Sum of the products of entries [q0, q1), every TEAM-th from the lane's,
+// AHEAD of them loaded at a time.
+template <typename T, int TEAM, int AHEAD>
+__device__ __forceinline__ T small_row_part(int32_t q0, int32_t q1, int lane,
+                                            const int32_t* __restrict__ crd,
+                                            const T* __restrict__ vals,
+                                            const T* __restrict__ x) {
+  T s = 0;
+  for (int32_t p = q0 + lane; p < q1; p += AHEAD * TEAM) {
+    T v[AHEAD], xv[AHEAD];
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) {
+      // Entries past the end repeat the lane's first one and add nothing.
+      const int32_t q = p + u * TEAM < q1 ? p + u * TEAM : p;
+      v[u] = vals[q];
+      xv[u] = x[crd[q]];
+    }
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u)
+      if (p + u * TEAM < q1) s += v[u] * xv[u];
+  }
+  return s;
+}
+// Repeated entries cost loads too: a row of 34 entries takes 4 a lane of its
+// team, not 16.
+template <typename T, int TEAM>
+__device__ __forceinline__ T small_row_sum(int32_t q0, int32_t q1, int lane,
+                                           const int32_t* __restrict__ crd,
+                                           const T* __restrict__ vals,
+                                           const T* __restrict__ x) {
+  return q1 - q0 <= 4 * TEAM   ? small_row_part<T, TEAM, 4>(q0, q1, lane, crd, vals, x)
+         : q1 - q0 <= 8 * TEAM ? small_row_part<T, TEAM, 8>(q0, q1, lane, crd, vals, x)
+                               : small_row_part<T, TEAM, kSmallAhead>(q0, q1, lane, crd, vals, x);
+}
+
 template <typename T, int G>
 __global__ __launch_bounds__(kSmallThreads) void k_spmv_small(
     int32_t m, const int32_t* __restrict__ pos, const int32_t* __restrict__ crd,
     const T* __restrict__ vals, const T* __restrict__ x, T* __restrict__ y) {
   constexpr int kRows = kSmallThreads / G;
-  constexpr int kAhead = 4, kLongAhead = 16;
-  __shared__ int32_t s_long[kRows];
-  __shared__ T s_sum[kSmallThreads / kWave];
-  __shared__ int s_count;
+  constexpr int kTeams = kSmallThreads / kSmallTeam, kWaves = kSmallThreads / kWave;
+  constexpr int kAhead = 4;
+  __shared__ int32_t s_team[kRows], s_wave[kRows], s_all[kRows];
+  __shared__ T s_sum[kWaves];
+  __shared__ int s_count[3];
   const int tid = threadIdx.x, sub = tid % G, slot = tid / G;
-  const int64_t i = (int64_t)blockIdx.x * kRows + slot;
+  const int64_t row0 = blockIdx.x, stride = gridDim.x;
+  const int64_t i = row0 + slot * stride;
   const int32_t p0 = i < m ? pos[i] : 0, p1 = i < m ? pos[i + 1] : 0;
   const bool is_long = p1 - p0 > kSmallOwn * G;
-  if (tid == 0) s_count = 0;
+  if (tid < 3) s_count[tid] = 0;
   __syncthreads();
-  if (sub == 0 && is_long) s_long[atomicAdd(&s_count, 1)] = slot;
+  if (sub == 0 && is_long) {
+    if (p1 - p0 <= kSmallTeamRow)
+      s_team[atomicAdd(&s_count[0], 1)] = slot;
+    else if (p1 - p0 <= kSmallWaveRow)
+      s_wave[atomicAdd(&s_count[1], 1)] = slot;
+    else
+      s_all[atomicAdd(&s_count[2], 1)] = slot;
+  }
   T acc = 0;
   for (int32_t p = is_long ? p1 : p0 + sub; p < p1; p += kAhead * G) {
     T v[kAhead], xv[kAhead];
@@ -362,33 +414,56 @@ __global__ __launch_bounds__(kSmallThreads) void k_spmv_small(
   for (int off = G / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, G);
   if (sub == 0 && i < m && !is_long) y[i] = acc;
   __syncthreads();
-  // Each long row's sum does not depend on the order of the list.
-  for (int k = 0; k < s_count; ++k) {
-    const int64_t row = (int64_t)blockIdx.x * kRows + s_long[k];
-    const int32_t q0 = pos[row], q1 = pos[row + 1];
-    T s = 0;
-    for (int32_t p = q0 + tid; p < q1; p += kLongAhead * kSmallThreads) {
-      T v[kLongAhead], xv[kLongAhead];
+  // Each long row's sum does not depend on the order of the lists.  Waves
+  // take rows from the last wave on, teams from the first.
+  for (int k = tid / kSmallTeam; k < s_count[0]; k += kTeams) {
+    const int64_t row = row0 + s_team[k] * stride;
+    T s = small_row_sum<T, kSmallTeam>(pos[row], pos[row + 1], tid % kSmallTeam, crd, vals, x);
 #pragma unroll
-      for (int u = 0; u < kLongAhead; ++u) {
-        const int32_t q = p + u * kSmallThreads < q1 ? p + u * kSmallThreads : p;
-        v[u] = vals[q];
-        xv[u] = x[crd[q]];
-      }
-#pragma unroll
-      for (int u = 0; u < kLongAhead; ++u)
-        if (p + u * kSmallThreads < q1) s += v[u] * xv[u];
-    }
+    for (int off = kSmallTeam / 2; off > 0; off >>= 1) s += __shfl_xor(s, off, kSmallTeam);
+    if (tid % kSmallTeam == 0) y[row] = s;
+  }
+  for (int k = kWaves - 1 - tid / kWave; k < s_count[1]; k += kWaves) {
+    const int64_t row = row0 + s_wave[k] * stride;
+    T s = small_row_sum<T, kWave>(pos[row], pos[row + 1], tid % kWave, crd, vals, x);
+    s = wave_sum(s);
+    if (tid % kWave == 0) y[row] = s;
+  }
+  for (int k = 0; k < s_count[2]; ++k) {
+    const int64_t row = row0 + s_all[k] * stride;
+    T s = small_row_sum<T, kSmallThreads>(pos[row], pos[row + 1], tid, crd, vals, x);
     s = wave_sum(s);
     if (tid % kWave == 0) s_sum[tid / kWave] = s;
     __syncthreads();
     if (tid == 0) {
       T all = 0;
-      for (int w = 0; w < kSmallThreads / kWave; ++w) all += s_sum[w];
+      for (int w = 0; w < kWaves; ++w) all += s_sum[w];
       y[row] = all;
     }
     __syncthreads();
   }
+}
+
+// Where this form is taken; times are f64, this form against the merge path.
+//   Few entries: 1000 rows of 10 3.5 against 7.8 us, 8192 of 8 4.7 : 8.4.
+//     Long rows that lie together: 512 of 64 among 10,500 of 3 5.5 : 8.3, 30
+//     of 2000 4.1 : 7.4, a power law of 4000 rows 6.2 : 8.0 (with the whole
+//     workgroup taking one long row after another 804, 98 and 21 us).  The
+//     line at 65,536 entries is not where the two meet: 131,072 in rows of 8
+//     take 5.3 : 8.5.
+//   No row that one workgroup takes too long for: a row holds at most n
+//     entries (one each of its columns).  Rows of 16,384 entries 7.0 : 7.9
+//     (four of them) and 8.5 : 9.0 (one among 12,000 of 2), of 24,000 13.2 :
+//     9.7; in f32 24,000 take 8.6 : 9.5.
+//   Not too many rows, which lie apart in pos and y here: 250,000 rows 9.0 :
+//     9.6, 500,000 16.2 : 11.2.
+constexpr int64_t kSmallEntries = 1 << 16;
+constexpr int64_t kSmallRows = 1 << 18;
+template <typename T>
+bool small_spmv(const CsrView& a) {
+  const int64_t longest = a.nnz < a.n ? a.nnz : a.n;
+  return a.nnz <= kSmallEntries && a.m <= kSmallRows &&
+         longest <= (sizeof(T) == 8 ? 16384 : 24576);
 }
 
 // Lanes a row: about three entries of an average row to a lane.
@@ -396,7 +471,9 @@ template <typename T>
 void launch_spmv_small(const CsrView& a, const T* x, T* y, hipStream_t st) {
   int g = 2;
   while (g < 64 && (int64_t)g * 3 * a.m < a.nnz) g <<= 1;
-  const unsigned grid = (unsigned)(((int64_t)a.m * g + kSmallThreads - 1) / kSmallThreads);
+  const int64_t need = ((int64_t)a.m * g + kSmallThreads - 1) / kSmallThreads;
+  const int64_t spread = a.m < kSmallSpread ? a.m : kSmallSpread;
+  const unsigned grid = (unsigned)((need > spread ? need : spread) | 1);
 #define TH_SMALL(G)                                                            \
   case G:                                                                      \
     k_spmv_small<T, G><<<grid, kSmallThreads, 0, st>>>(a.m, a.pos, a.crd,      \
@@ -472,7 +549,7 @@ int run_spmv(const CsrView& a, const T* x, T* y, const taco_hip_schedule& s,
                "spmv: MERGE_PATH uses 256-thread workgroups");
     TH_REQUIRE(k == 2 || k == 4 || k == 6 || k == 8 || k == 12 || k == 16,
                "spmv: items_per_thread %d unsupported for MERGE_PATH", k);
-    if (a.nnz <= kSmallEntries && (int64_t)a.m <= 16 * kSmallEntries) {
+    if (small_spmv<T>(a)) {
       launch_spmv_small<T>(a, x, y, st);
       return 0;
     }
