@@ -28,13 +28,18 @@ def _counts(name):
         c[7] = 70_000
     elif name == "run_lengths":  # runs of 7 .. 66 carries
         c = np.repeat(np.array([14_000, 16_400, 18_500, 20_500, 131_000, 135_000], np.int32), 2)
+    elif name == "wave_edges":  # carry runs that end and start at slots 63, 64, 65 of 512 items
+        t = 512
+        c = np.array([64 * t - 1, 64 * t - 1, 63 * t - 1, 2 * t, t, 65 * t + 3, 0, 128 * t - 8, 9 * t,
+                      16 * t, 5, 129 * t], np.int32)
     else:  # few rows
         c = np.array([40_000, 0, 0, 40_000], np.int32)
     return c
 
 
 @pytest.mark.parametrize("dtype,tol", [("f64", 1e-12), ("f32", 1e-5)])
-@pytest.mark.parametrize("name", ["front", "back", "middle", "above", "run_lengths", "few"])
+@pytest.mark.parametrize("name", ["front", "back", "middle", "above", "run_lengths", "few",
+                                  "wave_edges"])
 def test_corners(name, dtype, tol):
     counts = _counts(name)
     A = W.csr_from_counts(len(counts), 150_000, counts, 21)
