@@ -171,19 +171,19 @@ struct ShortRows {
 // in lanes: this kernel uses no LDS, so twice as many waves stay resident as
 // with the general row kernel (whose long-row accumulators take 32 KB of
 // LDS per workgroup), and each wave stages the loads of kRowsTogether rows
-// at once.  Longer rows are flagged (mid and *any_mid, cleared before) for
-// k_spgemm_numeric_mid.
+// at once.  mid[i] says of every row whether it is longer and left to
+// k_spgemm_numeric_mid; *listed is cleared for k_spgemm_list_mid.
 __global__ __launch_bounds__(256) void k_spgemm_numeric_short(
     int32_t m, const int32_t* __restrict__ apos, const int32_t* __restrict__ acrd,
     const double* __restrict__ avals, int32_t nnz_a, const int32_t* __restrict__ bpos,
     const int32_t* __restrict__ bcrd, const double* __restrict__ bvals, int32_t nnz_b,
     const int32_t* __restrict__ cpos, double* __restrict__ cvals, uint8_t* __restrict__ mid,
-    int32_t* __restrict__ any_mid) {
+    int32_t* __restrict__ listed) {
   const int lane = (int)__lane_id();
   const int64_t stride = (int64_t)gridDim.x * kWavesPerBlock;
   const int64_t first = (int64_t)blockIdx.x * kWavesPerBlock +
                         __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
-  if (nnz_a == 0 || nnz_b == 0) return;  // C has no entries
+  if (first == 0 && lane == 0) *listed = 0;
   const TacoHipSortMasks sm;
   for (int64_t base = first; base < m; base += kRowsTogether * stride) {
     ShortRows<kRowsTogether, true> r;
@@ -192,13 +192,8 @@ __global__ __launch_bounds__(256) void k_spgemm_numeric_short(
     for (int q = 0; q < kRowsTogether; ++q) {
       if (!r.real[q]) continue;
       const int64_t i = base + q * stride;
-      if (r.total[q] > 64) {
-        if (lane == 0) {
-          mid[i] = 1;
-          *any_mid = 1;
-        }
-        continue;
-      }
+      if (lane == 0) mid[i] = r.total[q] > 64;
+      if (r.total[q] > 64) continue;
       const int32_t c0 = cpos[i];
       taco_hip_spgemm_row_sum_store(r.total[q], r.col[q], r.prod[q], c0, cpos[i + 1] - c0,
                                     cvals, &sm);
@@ -208,36 +203,95 @@ __global__ __launch_bounds__(256) void k_spgemm_numeric_short(
 
 // ---- rows of more than 64 candidates (or more than 64 A entries) ----
 //
-// One wave per row.  The rows are not listed: a workgroup takes mid_chunk(m)
-// consecutive rows, reads which of them are its own kind with one coalesced
-// load and deals them to its four waves in row order.  A list needs an
-// atomic per row on one counter: with 100,003 rows to list the short-row
-// kernels took 1.07 ms each, without the list 16 and 26 us.  Neighbouring
-// rows also stay together, so rows of a banded product find their B rows in
-// L1 and L2.
+// One wave per row.  The rows are listed kListRows at a time: a workgroup
+// finds those among its rows and appends them, in their order, with one
+// atomic.  (One atomic a row took 1.07 ms for 100,003 rows.)  The list is
+// dealt out in pieces of a row for each wave, piece p to workgroup p modulo
+// the grid, so that heavy rows that lie together, as after a sort by degree,
+// are worked on side by side: taking neighbouring rows in turn, a wave had
+// up to 64 of them (256 rows of 1000 A entries first in 1,000,000 rows,
+// 8,000 candidates each: compute 11.1 ms, now 1.07).  Within a workgroup the waves claim rows as they get done.
 
-// Rows a workgroup takes: 16384 workgroups or more (64 a CU) as soon as the
-// rows allow, so that the last ones level out (100,003 banded rows, 4
-// resident workgroups a CU: 542, 378 and 277 us with 64, 32 and 8 rows each);
-// at most 256, and at least two for each wave, whose second row's loads then
-// run under the first one.
-inline int32_t mid_chunk(int32_t m) {
-  int32_t c = 8;
-  while (c < 256 && (int64_t)c * 16384 < m) c <<= 1;
-  return c;
+// Rows that one workgroup lists at a time, a word of flags a thread.
+constexpr int kListRows = 1024;
+// Appends the rows row0 + 4 * threadIdx.x + q whose bit q is set in `which`
+// to list, kept in order.  The whole workgroup calls it.
+__device__ __forceinline__ void list_rows(uint32_t which, int32_t row0,
+                                          int32_t* __restrict__ list,
+                                          int32_t* __restrict__ count) {
+  __shared__ int32_t s_n[kWavesPerBlock], s_base;
+  const int lane = (int)__lane_id(), wave = (int)(threadIdx.x / kWave);
+  const int32_t mine = __popc(which);
+  const int32_t inc = taco_hip_wave_scan_add_i32(mine);
+  if (lane == kWave - 1) s_n[wave] = inc;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int32_t all = 0;
+    for (int w = 0; w < kWavesPerBlock; ++w) all += s_n[w];
+    s_base = all > 0 ? atomicAdd(count, all) : 0;
+  }
+  __syncthreads();
+  int32_t at = s_base + inc - mine;
+  for (int w = 0; w < wave; ++w) at += s_n[w];
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    if ((which >> q) & 1) list[at++] = row0 + 4 * (int32_t)threadIdx.x + q;
+  __syncthreads();  // s_n may be written again
 }
+
+// The rows that k_spgemm_numeric_short marked.  mid holds m bytes from a
+// multiple of 4 on, up to a multiple of 4.
+__global__ __launch_bounds__(256) void k_spgemm_list_mid(int32_t m,
+                                                         const uint32_t* __restrict__ mid,
+                                                         int32_t* __restrict__ list,
+                                                         int32_t* __restrict__ listed) {
+  const int32_t row0 = (int32_t)blockIdx.x * kListRows;
+  const int64_t r = (int64_t)row0 + 4 * threadIdx.x;
+  const uint32_t flags = r < m ? mid[r / 4] : 0u;
+  uint32_t which = 0;
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    which |= r + q < m && ((flags >> (8 * q)) & 0xFF) ? 1u << q : 0u;
+  list_rows(which, row0, list, listed);
+}
+
+// Grid of the kernels below: as many workgroups as are resident, 4 a CU by
+// the LDS of k_spgemm_numeric_mid.  Workgroups without a row cost about 1 ns
+// each (16,384 of them 16 us in a product of short rows alone, now 4), and
+// 100,003 banded rows take 198, 231, 201 and 213 us in k_spgemm_numeric_mid
+// and what goes with it at 1024, 1536, 2048 and 4096 workgroups.
+constexpr int kMidGrid = 1024;
 inline unsigned mid_grid(int32_t m) {
-  const int64_t c = mid_chunk(m);
-  return (unsigned)(((int64_t)m + c - 1) / c);
+  const int64_t pieces = ((int64_t)m + kWavesPerBlock - 1) / kWavesPerBlock;
+  return (unsigned)(pieces < kMidGrid ? (pieces > 0 ? pieces : 1) : kMidGrid);
 }
 
-// First row of this workgroup: workgroups go to the 8 XCDs round robin, so
-// workgroup b takes chunk (b % 8) * (n / 8) + b / 8 (the remainder of n / 8
-// at the end as it comes) and an XCD's chunks are neighbours.
-__device__ __forceinline__ int64_t mid_first_row(int32_t chunk) {
-  const uint32_t per = gridDim.x / 8, b = blockIdx.x;
-  const uint32_t c = b < per * 8 ? (b % 8) * per + b / 8 : b;
-  return (int64_t)c * chunk;
+// A workgroup's share of the list, claimed by its waves an entry at a time:
+// entry e is list[(e / 4 * grid + slot) * 4 + e % 4].  Workgroups go to the 8
+// XCDs round robin.  Where the waves have more than a row each, slots run
+// over kXcdRun pieces on one XCD before they go on to the next, so that
+// neighbouring rows find their B rows in its L2.
+constexpr int kXcdRun = 32;
+struct Share {
+  int32_t count, grid, slot;
+  __device__ __forceinline__ Share(int32_t n) : count(n), grid((int32_t)gridDim.x) {
+    const int32_t b = (int32_t)blockIdx.x, run = 8 * kXcdRun;
+    const bool runs = n / kWavesPerBlock >= grid && b < grid / run * run;
+    slot = runs ? b / run * run + b % 8 * kXcdRun + b % run / 8 : b;
+  }
+  // INT_MAX and more past the int32 range: no entry.
+  __device__ __forceinline__ int64_t at(int32_t e) const {
+    return ((int64_t)(e / kWavesPerBlock) * grid + slot) * kWavesPerBlock + e % kWavesPerBlock;
+  }
+  // No entry of the share from e's piece on is in the list.
+  __device__ __forceinline__ bool over(int32_t e) const {
+    return at(e) - e % kWavesPerBlock >= count;
+  }
+};
+__device__ __forceinline__ int32_t claim(int32_t* next) {
+  int32_t e = 0;
+  if (__lane_id() == 0) e = atomicAdd(next, 1);
+  return __builtin_amdgcn_readfirstlane(e);
 }
 
 __device__ __forceinline__ double readlane_f64(double v, int lane) {
@@ -356,23 +410,8 @@ __device__ __forceinline__ void add_in_order(bool valid, int32_t slot, double pr
     if (valid && t == k) atomicAdd(acc + slot, prod);
 }
 
-// The share of this wave among the lanes (rows) of `rows`, dealt in order.
-__device__ __forceinline__ uint64_t my_share(bool selected) {
-  const int lane = (int)__lane_id();
-  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
-  const uint64_t rows = __ballot(selected);
-  const int rank = __popcll(rows & ((1ull << lane) - 1));
-  return __ballot(selected && (rank & (kWavesPerBlock - 1)) == wave);
-}
-// Takes the lowest set bit; 63 when there is none.
-__device__ __forceinline__ int take_bit(uint64_t* bits) {
-  const int bit = *bits ? __ffsll((unsigned long long)*bits) - 1 : 63;
-  *bits &= *bits - 1;
-  return bit;
-}
-
-// Numeric pass over the rows that k_spgemm_numeric_short flags.  A row's
-// sums live in LDS, 8 KB a wave (20 waves a CU):
+// Numeric pass over the listed rows.  A row's
+// sums live in LDS, 8 KB a wave (16 waves a CU):
 //   columns spanning at most 1024: the sum of column c at c - (first column);
 //   at most 682 columns: sums by position, found by binary search over the
 //     row's columns, staged in LDS beside them;
@@ -381,116 +420,130 @@ __device__ __forceinline__ int take_bit(uint64_t* bits) {
 // A B row's products go to LDS in one float-add instruction (add_in_order);
 // one product after another with a wait for each, as these rows were summed
 // before, took 2.5 ms on 100,003 banded rows of about 330 candidates (now
-// 243 us: each row's chain of loads, 16 waves a CU).
+// 184 us: each row's chain of loads, at those 16 waves).
 constexpr int kMidLdsBytes = 8192;
 constexpr int kMidSlots = kMidLdsBytes / 8;
 constexpr int kMidStaged = kMidLdsBytes / 12;
 __global__ __launch_bounds__(256) void k_spgemm_numeric_mid(
-    int32_t m, int32_t chunk, const uint8_t* __restrict__ mid,
-    const int32_t* __restrict__ any_mid, const int32_t* __restrict__ apos, const int32_t* __restrict__ acrd,
+    const int32_t* __restrict__ list, const int32_t* __restrict__ listed,
+    const int32_t* __restrict__ apos, const int32_t* __restrict__ acrd,
     const double* __restrict__ avals, const int32_t* __restrict__ bpos,
     const int32_t* __restrict__ bcrd, const double* __restrict__ bvals, int32_t nnz_b,
     const int32_t* __restrict__ cpos, const int32_t* __restrict__ ccrd,
     double* __restrict__ cvals) {
   __shared__ double s_acc[kWavesPerBlock][kMidSlots];
-  if (*any_mid == 0) return;
+  __shared__ int32_t s_next;
+  const Share share(*listed);
+  if (share.over(0)) return;
+  if (threadIdx.x == 0) s_next = 0;
+  __syncthreads();
   const int lane = (int)__lane_id();
   double* acc = s_acc[threadIdx.x / kWave];
   int32_t* keys = (int32_t*)(acc + kMidStaged);
-  const int64_t r0 = mid_first_row(chunk);
-  for (int32_t sub = 0; sub < chunk; sub += kWave) {
-    // Lane l holds what row r0 + sub + l starts from.
-    const int64_t r = r0 + sub + lane;
-    const bool listed = sub + lane < chunk && r < m && mid[r] != 0;
-    int32_t ha0 = 0, ha1 = 0, hc0 = 0, hnc = 0, hfirst = 0, hlast = -1;
-    if (listed) {
-      ha0 = apos[r];
-      ha1 = apos[r + 1];
-      hc0 = cpos[r];
-      hnc = cpos[r + 1] - hc0;
-      if (hnc > 0) {
-        hfirst = ccrd[hc0];
-        hlast = ccrd[hc0 + hnc - 1];
+  // Lane l holds what entry 64 * batch + l of the share starts from.
+  int32_t batch = -1;
+  int32_t hrow = -1, ha0 = 0, ha1 = 0, hc0 = 0, hnc = 0, hfirst = 0, hlast = -1;
+  // The next entry with columns, as its lane; -1: none is left.
+  const auto take = [&]() {
+    for (;;) {
+      const int32_t e = claim(&s_next);
+      if (share.over(e)) return -1;
+      if (e / kWave != batch) {
+        batch = e / kWave;
+        const int64_t q = share.at(batch * kWave + lane);
+        hrow = q < share.count ? list[q] : -1;
+        hnc = 0;
+        if (hrow >= 0) {
+          ha0 = apos[hrow];
+          ha1 = apos[hrow + 1];
+          hc0 = cpos[hrow];
+          hnc = cpos[hrow + 1] - hc0;
+          if (hnc > 0) {
+            hfirst = ccrd[hc0];
+            hlast = ccrd[hc0 + hnc - 1];
+          }
+        }
       }
+      if (__builtin_amdgcn_readlane(hnc, e % kWave) > 0) return e % kWave;
     }
-    uint64_t todo = my_share(listed && hnc > 0);
-    if (todo == 0) continue;
-    int bit = take_bit(&todo);
-    ARow<true> next;
-    next.entries(__builtin_amdgcn_readlane(ha0, bit), __builtin_amdgcn_readlane(ha1, bit), acrd,
-                 avals);
-    next.bounds(bpos);
-    for (bool more = true; more;) {
-      const ARow<true> row = next;
-      const int here = bit;
-      more = todo != 0;
-      if (more) bit = take_bit(&todo);
-      const int32_t c0 = __builtin_amdgcn_readlane(hc0, here);
-      const int32_t nc = __builtin_amdgcn_readlane(hnc, here);
-      const int32_t first = __builtin_amdgcn_readlane(hfirst, here);
-      const int64_t span = (int64_t)__builtin_amdgcn_readlane(hlast, here) - first + 1;
-      // The last row's successor is that row again.
-      next.entries(__builtin_amdgcn_readlane(ha0, bit), __builtin_amdgcn_readlane(ha1, bit),
-                   acrd, avals);
-      const auto bounds = [&]() { next.bounds(bpos); };
-      const int32_t* crow = ccrd + c0;
-      if (nc > kMidSlots) {
-        taco_hip_spgemm_row_numeric_global(apos, acrd, avals, bpos, bcrd, bvals,
-                                           (int32_t)(r0 + sub + here), c0, nc, ccrd, cvals);
-        bounds();
-      } else if (span > 0 && span <= kMidSlots) {
-        const uint32_t width = (uint32_t)span;
-        for (int q = lane; q < (int)width; q += kWave) acc[q] = 0.0;
-        taco_hip_wave_lds_sync();
-        for_each_candidate<true>(
-            row, acrd, avals, bpos, bcrd, bvals, nnz_b, bounds,
-            [&](bool valid, int32_t col, double prod, int32_t t) {
-              const uint32_t slot = (uint32_t)col - (uint32_t)first;
-              add_in_order(valid && slot < width, (int32_t)slot, prod, t, acc);
-            });
-        taco_hip_wave_lds_sync();
-        for (int q = lane; q < nc; q += kWave) {
-          const uint32_t slot = (uint32_t)crow[q] - (uint32_t)first;
-          __builtin_nontemporal_store(slot < width ? acc[slot] : 0.0, cvals + c0 + q);
-        }
-        taco_hip_wave_lds_sync();
-      } else {
-        const bool staged = nc <= kMidStaged;
-        for (int q = lane; q < nc; q += kWave) {
-          acc[q] = 0.0;
-          if (staged) keys[q] = crow[q];
-        }
-        taco_hip_wave_lds_sync();
-        int top = 1;  // the largest power of two <= nc
-        while (2 * top <= nc) top <<= 1;
-        for_each_candidate<true>(
-            row, acrd, avals, bpos, bcrd, bvals, nnz_b, bounds,
-            [&](bool valid, int32_t col, double prod, int32_t t) {
-              // The last position whose column is <= col.
-              int at = 0;
-              bool found;
-              if (staged) {
-                for (int step = top; step > 0; step >>= 1) {
-                  const int q = at + step < nc ? at + step : nc - 1;
-                  const int32_t key = keys[q];
-                  at = at + step < nc && key <= col ? q : at;
-                }
-                found = keys[at] == col;
-              } else {
-                for (int step = top; step > 0; step >>= 1) {
-                  const int q = at + step < nc ? at + step : nc - 1;
-                  const int32_t key = crow[q];
-                  at = at + step < nc && key <= col ? q : at;
-                }
-                found = crow[at] == col;
-              }
-              add_in_order(valid && found, at, prod, t, acc);
-            });
-        taco_hip_wave_lds_sync();
-        for (int q = lane; q < nc; q += kWave)
-          __builtin_nontemporal_store(acc[q], cvals + c0 + q);
-        taco_hip_wave_lds_sync();
+  };
+  int from = take();
+  if (from < 0) return;
+  int32_t a0 = __builtin_amdgcn_readlane(ha0, from), a1 = __builtin_amdgcn_readlane(ha1, from);
+  ARow<true> next;
+  next.entries(a0, a1, acrd, avals);
+  next.bounds(bpos);
+  while (from >= 0) {
+    const ARow<true> row = next;
+    const int32_t i = __builtin_amdgcn_readlane(hrow, from);
+    const int32_t c0 = __builtin_amdgcn_readlane(hc0, from);
+    const int32_t nc = __builtin_amdgcn_readlane(hnc, from);
+    const int32_t first = __builtin_amdgcn_readlane(hfirst, from);
+    const int64_t span = (int64_t)__builtin_amdgcn_readlane(hlast, from) - first + 1;
+    from = take();
+    if (from >= 0) {  // the last row's successor is that row again
+      a0 = __builtin_amdgcn_readlane(ha0, from);
+      a1 = __builtin_amdgcn_readlane(ha1, from);
+    }
+    next.entries(a0, a1, acrd, avals);
+    const auto bounds = [&]() { next.bounds(bpos); };
+    const int32_t* crow = ccrd + c0;
+    if (nc > kMidSlots) {
+      taco_hip_spgemm_row_numeric_global(apos, acrd, avals, bpos, bcrd, bvals,
+                                         i, c0, nc, ccrd, cvals);
+      bounds();
+    } else if (span > 0 && span <= kMidSlots) {
+      const uint32_t width = (uint32_t)span;
+      for (int q = lane; q < (int)width; q += kWave) acc[q] = 0.0;
+      taco_hip_wave_lds_sync();
+      for_each_candidate<true>(
+          row, acrd, avals, bpos, bcrd, bvals, nnz_b, bounds,
+          [&](bool valid, int32_t col, double prod, int32_t t) {
+            const uint32_t slot = (uint32_t)col - (uint32_t)first;
+            add_in_order(valid && slot < width, (int32_t)slot, prod, t, acc);
+          });
+      taco_hip_wave_lds_sync();
+      for (int q = lane; q < nc; q += kWave) {
+        const uint32_t slot = (uint32_t)crow[q] - (uint32_t)first;
+        __builtin_nontemporal_store(slot < width ? acc[slot] : 0.0, cvals + c0 + q);
       }
+      taco_hip_wave_lds_sync();
+    } else {
+      const bool staged = nc <= kMidStaged;
+      for (int q = lane; q < nc; q += kWave) {
+        acc[q] = 0.0;
+        if (staged) keys[q] = crow[q];
+      }
+      taco_hip_wave_lds_sync();
+      int top = 1;  // the largest power of two <= nc
+      while (2 * top <= nc) top <<= 1;
+      for_each_candidate<true>(
+          row, acrd, avals, bpos, bcrd, bvals, nnz_b, bounds,
+          [&](bool valid, int32_t col, double prod, int32_t t) {
+            // The last position whose column is <= col.
+            int at = 0;
+            bool found;
+            if (staged) {
+              for (int step = top; step > 0; step >>= 1) {
+                const int q = at + step < nc ? at + step : nc - 1;
+                const int32_t key = keys[q];
+                at = at + step < nc && key <= col ? q : at;
+              }
+              found = keys[at] == col;
+            } else {
+              for (int step = top; step > 0; step >>= 1) {
+                const int q = at + step < nc ? at + step : nc - 1;
+                const int32_t key = crow[q];
+                at = at + step < nc && key <= col ? q : at;
+              }
+              found = crow[at] == col;
+            }
+            add_in_order(valid && found, at, prod, t, acc);
+          });
+      taco_hip_wave_lds_sync();
+      for (int q = lane; q < nc; q += kWave)
+        __builtin_nontemporal_store(acc[q], cvals + c0 + q);
+      taco_hip_wave_lds_sync();
     }
   }
 }
@@ -525,16 +578,17 @@ __global__ __launch_bounds__(256) void k_spgemm_row_cands(
 
 // Pass 2 over the rows of at most 64 candidates (no LDS, so more waves stay
 // resident): each row's sorted distinct columns go to its scratch region
-// and its distinct count to counts.  Longer rows are left to
-// k_spgemm_symbolic_mid (status[5] set).  status[0] bit 4: the scratch holds fewer entries
-// than the candidate total, or the candidate offsets overflowed (nothing
-// done).
+// and its distinct count to counts.  Longer rows are first listed for
+// k_spgemm_symbolic_mid in mid_rows (status[5] of them), the rows of A
+// entries without candidates aside.  status[0] bit 4: the scratch holds
+// fewer entries than the candidate total, or the candidate offsets
+// overflowed (nothing done).
 __global__ __launch_bounds__(256) void k_spgemm_symbolic_short(
     int32_t m, const int32_t* __restrict__ apos, const int32_t* __restrict__ acrd,
     int32_t nnz_a, const int32_t* __restrict__ bpos, const int32_t* __restrict__ bcrd,
     int32_t nnz_b, const int32_t* __restrict__ candoff, int64_t capacity,
     int32_t* __restrict__ scratch, int32_t* __restrict__ counts,
-    int32_t* __restrict__ status) {
+    int32_t* __restrict__ mid_rows, int32_t* __restrict__ status) {
   const int lane = (int)__lane_id();
   const int64_t first = (int64_t)blockIdx.x * kWavesPerBlock +
                         __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
@@ -552,6 +606,23 @@ __global__ __launch_bounds__(256) void k_spgemm_symbolic_short(
       if (lane == 0) counts[i] = 0;
     return;
   }
+  for (int64_t row0 = (int64_t)blockIdx.x * kListRows; row0 < m;
+       row0 += (int64_t)gridDim.x * kListRows) {
+    uint32_t which = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int64_t r = row0 + 4 * threadIdx.x + q;
+      if (r >= m) continue;
+      const int32_t n = candoff[r + 1] - candoff[r];
+      if (n > 64 || apos[r + 1] - apos[r] > 64) {
+        if (n > 0)
+          which |= 1u << q;
+        else
+          counts[r] = 0;
+      }
+    }
+    list_rows(which, (int32_t)row0, mid_rows, status + 5);
+  }
   const TacoHipSortMasks sm;
   for (int64_t base = first; base < m; base += kRowsTogether * stride) {
     ShortRows<kRowsTogether, false> r;
@@ -560,10 +631,7 @@ __global__ __launch_bounds__(256) void k_spgemm_symbolic_short(
     for (int q = 0; q < kRowsTogether; ++q) {
       if (!r.real[q]) continue;
       const int64_t i = base + q * stride;
-      if (r.total[q] > 64) {
-        if (lane == 0) status[5] = 1;
-        continue;
-      }
+      if (r.total[q] > 64) continue;
       const int32_t v = (int32_t)taco_hip_wave_sort_u32((uint32_t)r.col[q], sm);
       const int32_t prev = __shfl_up(v, 1, 64);
       const bool head = v != INT_MAX && (lane == 0 || prev != v);
@@ -649,7 +717,7 @@ __device__ __forceinline__ int32_t sort_distinct(const int32_t* buf, int32_t n, 
 //   otherwise: the LDS hash set of up to TACO_HIP_ROW_CAP distinct columns
 //     (rows beyond it are listed in long_rows, status[1], for the
 //     global-memory sort, their count left 0).
-// Flags and bits need no sort and cost nothing for a repeated column: 154 us
+// Flags and bits need no sort and cost nothing for a repeated column: 123 us
 // on 100,003 banded rows of about 330 candidates and 245 columns, where the
 // hash set with its 1024-entry sort through LDS, which every such row took
 // before, took 2.67 ms.  A B
@@ -657,154 +725,165 @@ __device__ __forceinline__ int32_t sort_distinct(const int32_t* buf, int32_t n, 
 // is noticed and goes to the hash set.
 constexpr int kMidFlags = TACO_HIP_ROW_CAP;
 __global__ __launch_bounds__(256) void k_spgemm_symbolic_mid(
-    int32_t m, int32_t chunk, const int32_t* __restrict__ apos,
+    const int32_t* __restrict__ mid_rows, const int32_t* __restrict__ apos,
     const int32_t* __restrict__ acrd, const int32_t* __restrict__ bpos,
     const int32_t* __restrict__ bcrd, int32_t nnz_b, const int32_t* __restrict__ candoff,
     int32_t* __restrict__ scratch, int32_t* __restrict__ counts,
     int32_t* __restrict__ long_rows, int32_t* __restrict__ status) {
   __shared__ TacoHipRowSet s_sets[kWavesPerBlock];
-  if ((status[0] & 4) || status[5] == 0) return;
+  __shared__ int32_t s_next;
+  const Share share(status[0] & 4 ? 0 : status[5]);
+  if (share.over(0)) return;
+  if (threadIdx.x == 0) s_next = 0;
+  __syncthreads();
   const int lane = (int)__lane_id();
   TacoHipRowSet* w = &s_sets[threadIdx.x / kWave];
   int32_t* buf = w->keys;
-  const int64_t r0 = mid_first_row(chunk);
-  for (int32_t sub = 0; sub < chunk; sub += kWave) {
-    // Lane l holds what row r0 + sub + l starts from.
-    const int64_t r = r0 + sub + lane;
-    int32_t ha0 = 0, ha1 = 0, hoff = 0, hn = 0;
-    if (sub + lane < chunk && r < m) {
-      ha0 = apos[r];
-      ha1 = apos[r + 1];
-      hoff = candoff[r];
-      hn = candoff[r + 1] - hoff;
+  // Lane l holds what entry 64 * batch + l of the share starts from.
+  int32_t batch = -1;
+  int32_t hrow = -1, ha0 = 0, ha1 = 0, hoff = 0, hn = 0;
+  // The next entry, as its lane; -1: none is left.
+  const auto take = [&]() {
+    for (;;) {
+      const int32_t e = claim(&s_next);
+      if (share.over(e)) return -1;
+      if (e / kWave != batch) {
+        batch = e / kWave;
+        const int64_t q = share.at(batch * kWave + lane);
+        hrow = q < share.count ? mid_rows[q] : -1;
+        if (hrow >= 0) {
+          ha0 = apos[hrow];
+          ha1 = apos[hrow + 1];
+          hoff = candoff[hrow];
+          hn = candoff[hrow + 1] - hoff;
+        }
+      }
+      if (__builtin_amdgcn_readlane(hrow, e % kWave) >= 0) return e % kWave;
     }
-    const bool mid = hn > 64 || ha1 - ha0 > 64;
-    if (mid && hn == 0) counts[r] = 0;  // every wave stores the same
-    uint64_t todo = my_share(mid && hn > 0);
-    if (todo == 0) continue;
-    int bit = take_bit(&todo);
-    // The next row's entries, bounds, and the ends of its B rows.
-    ARow<false> next;
-    int32_t lo, hi;
-    const auto ends = [&]() {
-      next.bounds(bpos);
-      const int32_t k = next.n > 0 ? next.b0 : 0;
-      const int32_t f = bcrd[k], l = bcrd[next.n > 0 ? next.b0 + next.n - 1 : 0];
-      lo = next.n > 0 ? f : INT_MAX;
-      hi = next.n > 0 ? l : -1;
-    };
-    next.entries(__builtin_amdgcn_readlane(ha0, bit), __builtin_amdgcn_readlane(ha1, bit), acrd,
-                 nullptr);
-    ends();
-    for (bool more = true; more;) {
-      const ARow<false> row = next;
-      const int here = bit;
-      more = todo != 0;
-      if (more) bit = take_bit(&todo);
-      const int32_t i = (int32_t)(r0 + sub + here);
-      const int32_t n = __builtin_amdgcn_readlane(hn, here);
-      int32_t* dst = scratch + __builtin_amdgcn_readlane(hoff, here);
-      // A's entries past the first 64.
-      for (int32_t p = row.a0 + kWave + lane; p < row.a0 + row.la; p += kWave) {
-        const int32_t j = acrd[p];
-        const int32_t b0 = bpos[j], b1 = bpos[j + 1];
-        if (b0 < b1) {
-          const int32_t f = bcrd[b0], l = bcrd[b1 - 1];
-          lo = f < lo ? f : lo;
-          hi = l > hi ? l : hi;
-        }
+  };
+  int from = take();
+  if (from < 0) return;
+  // The next row's entries, bounds, and the ends of its B rows.
+  ARow<false> next;
+  int32_t lo, hi;
+  const auto ends = [&]() {
+    next.bounds(bpos);
+    const int32_t k = next.n > 0 ? next.b0 : 0;
+    const int32_t f = bcrd[k], l = bcrd[next.n > 0 ? next.b0 + next.n - 1 : 0];
+    lo = next.n > 0 ? f : INT_MAX;
+    hi = next.n > 0 ? l : -1;
+  };
+  int32_t a0 = __builtin_amdgcn_readlane(ha0, from), a1 = __builtin_amdgcn_readlane(ha1, from);
+  next.entries(a0, a1, acrd, nullptr);
+  ends();
+  while (from >= 0) {
+    const ARow<false> row = next;
+    const int32_t i = __builtin_amdgcn_readlane(hrow, from);
+    const int32_t n = __builtin_amdgcn_readlane(hn, from);
+    int32_t* dst = scratch + __builtin_amdgcn_readlane(hoff, from);
+    from = take();
+    if (from >= 0) {  // the last row's successor is that row again
+      a0 = __builtin_amdgcn_readlane(ha0, from);
+      a1 = __builtin_amdgcn_readlane(ha1, from);
+    }
+    // A's entries past the first 64.
+    for (int32_t p = row.a0 + kWave + lane; p < row.a0 + row.la; p += kWave) {
+      const int32_t j = acrd[p];
+      const int32_t b0 = bpos[j], b1 = bpos[j + 1];
+      if (b0 < b1) {
+        const int32_t f = bcrd[b0], l = bcrd[b1 - 1];
+        lo = f < lo ? f : lo;
+        hi = l > hi ? l : hi;
       }
+    }
 #pragma unroll
-      for (int off = 32; off > 0; off >>= 1) {
-        const int32_t a = __shfl_xor(lo, off, 64), b = __shfl_xor(hi, off, 64);
-        lo = a < lo ? a : lo;
-        hi = b > hi ? b : hi;
-      }
-      const int32_t low = __builtin_amdgcn_readfirstlane(lo);
-      const int64_t span64 = (int64_t)__builtin_amdgcn_readfirstlane(hi) - low + 1;
-      // The last row's successor is that row again.
-      next.entries(__builtin_amdgcn_readlane(ha0, bit), __builtin_amdgcn_readlane(ha1, bit),
-                   acrd, nullptr);
-      int32_t cnt = -1;
-      if (span64 > 0 && span64 <= kMidFlags) {
-        const uint32_t span = (uint32_t)span64;
-        for (int q = lane; q < (int)span; q += kWave) buf[q] = 0;
-        taco_hip_wave_lds_sync();
-        bool outside = false;
-        for_each_candidate<false>(row, acrd, nullptr, bpos, bcrd, nullptr, nnz_b, ends,
-                                  [&](bool, int32_t col, double, int32_t) {
-                                    // Lanes past the end repeat a column.
-                                    const uint32_t at = (uint32_t)col - (uint32_t)low;
-                                    if (at < span) buf[at] = 1;
-                                    outside |= at >= span;
-                                  });
-        taco_hip_wave_lds_sync();
-        if (__ballot(outside) == 0) {
-          cnt = 0;
-          for (int q0 = 0; q0 < (int)span; q0 += kWave) {
-            const int q = q0 + lane;
-            const bool set = q < (int)span && buf[q] != 0;
-            const uint64_t mask = __ballot(set);
-            if (set) dst[cnt + __popcll(mask & ((1ull << lane) - 1))] = low + q;
-            cnt += __popcll(mask);
-          }
-        }
-        taco_hip_wave_lds_sync();
-      } else if (span64 > 0 && span64 <= 32 * kMidFlags) {
-        const uint32_t span = (uint32_t)span64;
-        const int words = (int)((span + 31) / 32);
-        for (int q = lane; q < words; q += kWave) buf[q] = 0;
-        taco_hip_wave_lds_sync();
-        bool outside = false;
-        for_each_candidate<false>(row, acrd, nullptr, bpos, bcrd, nullptr, nnz_b, ends,
-                                  [&](bool valid, int32_t col, double, int32_t) {
-                                    const uint32_t at = (uint32_t)col - (uint32_t)low;
-                                    if (valid && at < span)
-                                      atomicOr(buf + (at >> 5), 1 << (at & 31));
-                                    outside |= valid && at >= span;
-                                  });
-        taco_hip_wave_lds_sync();
-        if (__ballot(outside) == 0) {
-          const int per = (words + kWave - 1) / kWave;  // consecutive words a lane
-          const int w0 = lane * per, w1 = w0 + per < words ? w0 + per : words;
-          int32_t held = 0;
-          for (int q = w0; q < w1; ++q) held += __popc((uint32_t)buf[q]);
-          const int32_t inc = taco_hip_wave_scan_add_i32(held);
-          int32_t at = inc - held;
-          for (int q = w0; q < w1; ++q)
-            for (uint32_t b = (uint32_t)buf[q]; b; b &= b - 1)
-              dst[at++] = low + 32 * q + (__ffs((int)b) - 1);
-          cnt = __builtin_amdgcn_readlane(inc, 63);
-        }
-        taco_hip_wave_lds_sync();
-      } else if (n <= TACO_HIP_ROW_CAP) {
-        int32_t at = 0;
-        for_each_candidate<false>(row, acrd, nullptr, bpos, bcrd, nullptr, nnz_b, ends,
-                                  [&](bool valid, int32_t col, double, int32_t) {
-                                    if (valid) buf[at + lane] = col;
-                                    at += __popcll(__ballot(valid));
-                                  });
-        taco_hip_wave_lds_sync();
-        cnt = n <= 128   ? sort_distinct<2>(buf, n, dst)
-              : n <= 256 ? sort_distinct<4>(buf, n, dst)
-              : n <= 512 ? sort_distinct<8>(buf, n, dst)
-                         : sort_distinct<16>(buf, n, dst);
-        taco_hip_wave_lds_sync();
-      } else {
-        ends();
-      }
-      if (cnt < 0) {
-        cnt = taco_hip_row_hash(w, apos, acrd, bpos, bcrd, i);
-        if (cnt >= 0) {
-          taco_hip_row_hash_sort(w);
-          for (int q = lane; q < cnt; q += kWave) dst[q] = buf[q];
-          taco_hip_wave_lds_sync();
+    for (int off = 32; off > 0; off >>= 1) {
+      const int32_t a = __shfl_xor(lo, off, 64), b = __shfl_xor(hi, off, 64);
+      lo = a < lo ? a : lo;
+      hi = b > hi ? b : hi;
+    }
+    const int32_t low = __builtin_amdgcn_readfirstlane(lo);
+    const int64_t span64 = (int64_t)__builtin_amdgcn_readfirstlane(hi) - low + 1;
+    next.entries(a0, a1, acrd, nullptr);
+    int32_t cnt = -1;
+    if (span64 > 0 && span64 <= kMidFlags) {
+      const uint32_t span = (uint32_t)span64;
+      for (int q = lane; q < (int)span; q += kWave) buf[q] = 0;
+      taco_hip_wave_lds_sync();
+      bool outside = false;
+      for_each_candidate<false>(row, acrd, nullptr, bpos, bcrd, nullptr, nnz_b, ends,
+                                [&](bool, int32_t col, double, int32_t) {
+                                  // Lanes past the end repeat a column.
+                                  const uint32_t at = (uint32_t)col - (uint32_t)low;
+                                  if (at < span) buf[at] = 1;
+                                  outside |= at >= span;
+                                });
+      taco_hip_wave_lds_sync();
+      if (__ballot(outside) == 0) {
+        cnt = 0;
+        for (int q0 = 0; q0 < (int)span; q0 += kWave) {
+          const int q = q0 + lane;
+          const bool set = q < (int)span && buf[q] != 0;
+          const uint64_t mask = __ballot(set);
+          if (set) dst[cnt + __popcll(mask & ((1ull << lane) - 1))] = low + q;
+          cnt += __popcll(mask);
         }
       }
-      if (lane == 0) {
-        if (cnt < 0) long_rows[atomicAdd(status + 1, 1)] = i;
-        counts[i] = cnt < 0 ? 0 : cnt;
+      taco_hip_wave_lds_sync();
+    } else if (span64 > 0 && span64 <= 32 * kMidFlags) {
+      const uint32_t span = (uint32_t)span64;
+      const int words = (int)((span + 31) / 32);
+      for (int q = lane; q < words; q += kWave) buf[q] = 0;
+      taco_hip_wave_lds_sync();
+      bool outside = false;
+      for_each_candidate<false>(row, acrd, nullptr, bpos, bcrd, nullptr, nnz_b, ends,
+                                [&](bool valid, int32_t col, double, int32_t) {
+                                  const uint32_t at = (uint32_t)col - (uint32_t)low;
+                                  if (valid && at < span)
+                                    atomicOr(buf + (at >> 5), 1 << (at & 31));
+                                  outside |= valid && at >= span;
+                                });
+      taco_hip_wave_lds_sync();
+      if (__ballot(outside) == 0) {
+        const int per = (words + kWave - 1) / kWave;  // consecutive words a lane
+        const int w0 = lane * per, w1 = w0 + per < words ? w0 + per : words;
+        int32_t held = 0;
+        for (int q = w0; q < w1; ++q) held += __popc((uint32_t)buf[q]);
+        const int32_t inc = taco_hip_wave_scan_add_i32(held);
+        int32_t at = inc - held;
+        for (int q = w0; q < w1; ++q)
+          for (uint32_t b = (uint32_t)buf[q]; b; b &= b - 1)
+            dst[at++] = low + 32 * q + (__ffs((int)b) - 1);
+        cnt = __builtin_amdgcn_readlane(inc, 63);
       }
+      taco_hip_wave_lds_sync();
+    } else if (n <= TACO_HIP_ROW_CAP) {
+      int32_t at = 0;
+      for_each_candidate<false>(row, acrd, nullptr, bpos, bcrd, nullptr, nnz_b, ends,
+                                [&](bool valid, int32_t col, double, int32_t) {
+                                  if (valid) buf[at + lane] = col;
+                                  at += __popcll(__ballot(valid));
+                                });
+      taco_hip_wave_lds_sync();
+      cnt = n <= 128   ? sort_distinct<2>(buf, n, dst)
+            : n <= 256 ? sort_distinct<4>(buf, n, dst)
+            : n <= 512 ? sort_distinct<8>(buf, n, dst)
+                       : sort_distinct<16>(buf, n, dst);
+      taco_hip_wave_lds_sync();
+    } else {
+      ends();
+    }
+    if (cnt < 0) {
+      cnt = taco_hip_row_hash(w, apos, acrd, bpos, bcrd, i);
+      if (cnt >= 0) {
+        taco_hip_row_hash_sort(w);
+        for (int q = lane; q < cnt; q += kWave) dst[q] = buf[q];
+        taco_hip_wave_lds_sync();
+      }
+    }
+    if (lane == 0) {
+      if (cnt < 0) long_rows[atomicAdd(status + 1, 1)] = i;
+      counts[i] = cnt < 0 ? 0 : cnt;
     }
   }
 }
@@ -1165,9 +1244,9 @@ int assemble_two_pass(const CsrView& a, const CsrView& b, taco_tensor_t* C,
   return rc;
 }
 
-// Workspace slots of the one-sort assemble, and of compute's row flags.
+// Workspace slots of the one-sort assemble, and of compute's rows.
 constexpr int kSlotCandOff = 8, kSlotScratch = 9, kSlotLongMeta = 10, kSlotLongKeys = 11,
-              kSlotSortTemp = 12, kSlotComputeFlags = 13;
+              kSlotSortTemp = 12, kSlotComputeRows = 13;
 // Workgroups per CU of k_spgemm_numeric_short's resident grid.
 constexpr int kShortBlocksPerCu = 8;
 
@@ -1249,14 +1328,15 @@ int assemble_one_sort(const CsrView& a, const CsrView& b, taco_tensor_t* C, hipS
   const int32_t m = a.m;
   // status[0]: flags (2: nnz(C) beyond int32, 4: scratch too small);
   // status[1]: long rows listed; status[2]: candidate-total flags (2);
-  // status[3]: candidates; status[4]: nnz(C); status[5]: not 0 if any row has
+  // status[3]: candidates; status[4]: nnz(C); status[5]: rows of
   // more than 64 candidates or A entries.
-  char* ws = (char*)workspace(256 + sizeof(int32_t) * 2 * ((size_t)m + 1), 2);
+  char* ws = (char*)workspace(256 + sizeof(int32_t) * 3 * ((size_t)m + 1), 2);
   int32_t* candoff = (int32_t*)workspace(sizeof(int32_t) * ((size_t)m + 1), kSlotCandOff);
   if (!ws || !candoff) return 1;
   int32_t* status = (int32_t*)ws;
   int32_t* counts = (int32_t*)(ws + 256);
   int32_t* long_rows = counts + m + 1;
+  int32_t* mid_rows = long_rows + m + 1;
   int32_t* cpos = (int32_t*)taco_hip_unified_alloc(sizeof(int32_t) * ((size_t)m + 1));
   if (!cpos) return 1;
   const unsigned short_grid = short_rows_grid(m);
@@ -1288,10 +1368,10 @@ int assemble_one_sort(const CsrView& a, const CsrView& b, taco_tensor_t* C, hipS
       if (m > 0) {
         k_spgemm_symbolic_short<<<short_grid, 256, 0, st>>>(
             m, a.pos, a.crd, (int32_t)a.nnz, b.pos, b.crd, (int32_t)b.nnz, candoff,
-            (int64_t)(cap_bytes / sizeof(int32_t)), scratch, counts, status);
+            (int64_t)(cap_bytes / sizeof(int32_t)), scratch, counts, mid_rows, status);
         k_spgemm_symbolic_mid<<<mid_grid(m), 256, 0, st>>>(
-            m, mid_chunk(m), a.pos, a.crd, b.pos, b.crd, (int32_t)b.nnz, candoff, scratch,
-            counts, long_rows, status);
+            mid_rows, a.pos, a.crd, b.pos, b.crd, (int32_t)b.nnz, candoff, scratch, counts,
+            long_rows, status);
       }
       if ((rc = device_counts_to_pos(m, counts, cpos, status, st, status + 4))) break;
       if ((rc = read_back_i32(status, 5, host, st))) break;
@@ -1367,20 +1447,23 @@ extern "C" int taco_hip_spgemm_compute(taco_tensor_t* C, taco_tensor_t* A,
   if (int rc = view_csr(C, "C", &c)) return rc;
   if (a.m == 0 || c.nnz == 0) return finish("taco_hip_spgemm_compute");
   hipStream_t st = current_stream();
-  // Workspace: whether any row has more than 64 candidates, then a flag per
-  // row for those that do.
-  const size_t flag_bytes = sizeof(int32_t) + ((size_t)a.m + 3) / 4 * 4;
-  int32_t* any_mid = (int32_t*)workspace(flag_bytes, kSlotComputeFlags);
-  if (!any_mid) return 1;
-  uint8_t* mid = (uint8_t*)(any_mid + 1);
-  if (int rc = zero_fill(any_mid, flag_bytes, st)) return rc;
+  if (a.nnz == 0 || b.nnz == 0) return finish("taco_hip_spgemm_compute");  // no products
+  // Workspace: the number of rows of more than 64 candidates, a list for
+  // them, and a flag for every row.
+  const size_t flag_bytes = ((size_t)a.m + 3) / 4 * 4;
+  int32_t* listed = (int32_t*)workspace(
+      256 + sizeof(int32_t) * (size_t)a.m + flag_bytes, kSlotComputeRows);
+  if (!listed) return 1;
+  int32_t* list = listed + 64;
+  uint8_t* mid = (uint8_t*)(list + a.m);
   k_spgemm_numeric_short<<<short_rows_grid(a.m), 256, 0, st>>>(
       a.m, a.pos, a.crd, (const double*)a.vals, (int32_t)a.nnz, b.pos, b.crd,
-      (const double*)b.vals, (int32_t)b.nnz, c.pos, (double*)c.vals, mid,
-      any_mid);
+      (const double*)b.vals, (int32_t)b.nnz, c.pos, (double*)c.vals, mid, listed);
+  k_spgemm_list_mid<<<(unsigned)(((int64_t)a.m + kListRows - 1) / kListRows), 256, 0, st>>>(
+      a.m, (const uint32_t*)mid, list, listed);
   k_spgemm_numeric_mid<<<mid_grid(a.m), 256, 0, st>>>(
-      a.m, mid_chunk(a.m), mid, any_mid, a.pos, a.crd, (const double*)a.vals, b.pos, b.crd,
-      (const double*)b.vals, (int32_t)b.nnz, c.pos, c.crd, (double*)c.vals);
+      list, listed, a.pos, a.crd, (const double*)a.vals, b.pos, b.crd, (const double*)b.vals,
+      (int32_t)b.nnz, c.pos, c.crd, (double*)c.vals);
   return finish("taco_hip_spgemm_compute");
 }
 

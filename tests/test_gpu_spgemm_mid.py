@@ -3,10 +3,14 @@ kernels (flags, bits, register sorts of 2 to 16 values a lane, hash set;
 sums by column, by staged and by unstaged search), at the edges between them,
 against the oracle: pos and crd bit for bit, and the values too, since every
 column sums separately rounded products in encounter order."""
+import ctypes
+
 import numpy as np
 import pytest
+import torch
 
 import oracle
+from taco_amd import _lib, descriptors as D
 from taco_amd import workloads as W
 from tests import gpu_util as G
 
@@ -93,3 +97,61 @@ def test_subnormal_sums():
     _, crd, vals = G.spgemm(A, B)
     assert crd.tolist() == [0, 1, 2]
     assert vals.view(np.int64).tolist() == k.reshape(70, 3).sum(0).tolist()
+
+
+def _check(A, B):
+    pos, crd, vals = G.spgemm(A, B)
+    opos, ocrd = oracle.spgemm_assemble(A, B)
+    assert np.array_equal(pos, opos) and np.array_equal(crd, ocrd)
+    assert np.array_equal(vals, oracle.spgemm_compute(A, B, opos, ocrd))
+
+
+@pytest.mark.parametrize("m", [1, 3, 4, 5, 1023, 1024, 1025, 4095, 4096, 4097, 8191, 65536, 70001])
+def test_every_row_listed(m):
+    """Row counts around what a workgroup lists at a time (1024), the resident
+    grid's waves (4096, past which neighbouring pieces stay on an XCD) and 64
+    entries of the list for each workgroup (65,536).  66 candidates a row."""
+    rng = np.random.default_rng(m)
+    B = _csr([np.sort(rng.choice(500, 33, replace=False)) for _ in range(90)], 500, m)
+    A = _csr(np.sort(np.stack([rng.integers(0, 45, m), rng.integers(45, 90, m)], 1), 1), 90, m + 1)
+    _check(A, B)
+
+
+@pytest.mark.parametrize("every", [1, 2, 7])
+def test_long_rows_without_products(every):
+    """Rows of more than 64 entries that all name empty rows of B, alone and
+    among rows with products."""
+    m, k = 1300, 200
+    B = _csr([[], *([[5, 9, 11]] * 99)] + [[]] * 100, 20, 3)
+    A = _csr([np.arange(100, 200) if i % every == 0 else np.arange(i % 100) for i in range(m)], k, 4)
+    _check(A, B)
+
+
+def test_heavy_rows_together_keep_their_pace():
+    """Heavy rows that lie together (an operand sorted by degree) take about
+    as long as the same rows spread out; with neighbouring
+    rows left to a wave, 6 times."""
+    m, heavy = 500_000, 256
+    B = W.csr_from_counts(m, m, np.full(m, 8, np.int32), 41, W.STRUCT_BANDED, 64)
+    took = {}
+    for name, rows in (("together", np.arange(heavy)),
+                       ("spread", np.arange(heavy) * (m // heavy))):
+        counts = np.ones(m, np.int32)
+        counts[rows] = 1000
+        A = W.csr_from_counts(m, 20_000, counts, 42)
+        A.n = m  # heavy rows name 20,000 of B's rows
+        a, b, c = G.csr_desc(A), G.csr_desc(B), D.csr_empty((m, m))
+        L = _lib.lib()
+        _lib.check(L.taco_hip_spgemm_assemble(c.ptr, a.ptr, b.ptr))
+        best = []
+        for _ in range(4):
+            t0, t1 = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            t0.record()
+            _lib.check(L.taco_hip_spgemm_compute(c.ptr, a.ptr, b.ptr))
+            t1.record()
+            torch.cuda.synchronize()
+            best.append(t0.elapsed_time(t1))
+        took[name] = min(best)
+        for p in (c.level_ptr(1, 0), c.level_ptr(1, 1), c.vals_ptr()):
+            L.taco_hip_unified_free(ctypes.c_void_p(p))
+    assert took["together"] < 3 * took["spread"], took

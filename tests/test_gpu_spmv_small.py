@@ -110,8 +110,8 @@ def _microseconds(A, x, sched, calls=100):
                          ids=["dense_block", "block_among_empty", "few_long", "many_short_long"])
 def test_long_rows_together_keep_their_pace(counts):
     """Long rows side by side are summed side by side: the default schedule
-    stays within 4 times an equal split of the entries (0.5 to 0.7 times;
-    one after another it was 12 to 110 times)."""
+    stays within 4 times an equal split of the entries (0.4 to 0.7 times;
+    one after another it was 5 to 90 times)."""
     A = W.csr_from_counts(len(counts), 16384, np.array(counts, np.int32), 31)
     x = W.uniform(A.n, 32, W.STREAM_X)
     split = _microseconds(A, x, G.sched(_lib.NNZ_SPLIT, 256, items=8))
