@@ -98,6 +98,31 @@ __device__ __forceinline__ void for_each_task(const Queues& qs, int32_t* s_slot,
   }
 }
 
+// The products of entries [c0, c1) to prod, AHEAD of them in flight for each
+// thread.
+template <int AHEAD>
+__device__ __forceinline__ void stream_products(const int32_t* __restrict__ ic,
+                                                const float* __restrict__ iv,
+                                                const float* __restrict__ ix, int32_t c0,
+                                                int32_t c1, float* prod) {
+  for (int32_t q = c0 + (int32_t)threadIdx.x; q < c1; q += AHEAD * kBatchThreads) {
+    int32_t j[AHEAD];
+    float v[AHEAD], xv[AHEAD];
+    // Entries past the chunk repeat its last one.
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) {
+      const int32_t e = q + u * kBatchThreads < c1 ? q + u * kBatchThreads : c1 - 1;
+      j[u] = stream_load(ic + e);
+      v[u] = stream_load(iv + e);
+    }
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) xv[u] = ix[j[u]];
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u)
+      if (q + u * kBatchThreads < c1) prod[q + u * kBatchThreads - c0] = v[u] * xv[u];
+  }
+}
+
 __global__ __launch_bounds__(kBatchThreads) void k_batch_spmv(
     Queues qs, const Task* __restrict__ tasks, const Inst* __restrict__ insts,
     const int32_t* __restrict__ pos, const int32_t* __restrict__ crd,
@@ -122,7 +147,9 @@ __global__ __launch_bounds__(kBatchThreads) void k_batch_spmv(
       // products.  Passes of kBatchThreads rows; rows longer than a chunk
       // span chunks.  With one entry and its gather at a time a chunk was 16
       // waits for memory in turn, now 2: 128 instances of 1,000 .. 200,000
-      // rows (4.8 M rows, 0.95 GB), 496 -> 412 us.
+      // rows (4.8 M rows, 0.95 GB), 479 -> 399 us.  A chunk of few entries has
+      // 2 or 4 of them in flight, since repeated ones cost loads too (rows of
+      // 2 .. 4 entries, 2.6 M: 84.7 us with 8, now 78.1).
       for (int32_t rb = tk.r0; rb < tk.r1; rb += kBatchThreads) {
         const int32_t re_ = rb + kBatchThreads < tk.r1 ? rb + kBatchThreads : tk.r1;
         const int32_t r = rb + tid;
@@ -131,22 +158,12 @@ __global__ __launch_bounds__(kBatchThreads) void k_batch_spmv(
         float acc = 0.f;
         for (int32_t c0 = e_begin; c0 < e_end; c0 += kStreamChunk) {
           const int32_t c1 = c0 + kStreamChunk < e_end ? c0 + kStreamChunk : e_end;
-          for (int32_t q = c0 + tid; q < c1; q += kStreamAhead * kBatchThreads) {
-            int32_t j[kStreamAhead];
-            float v[kStreamAhead], xv[kStreamAhead];
-            // Entries past the chunk repeat its last one.
-#pragma unroll
-            for (int u = 0; u < kStreamAhead; ++u) {
-              const int32_t e = q + u * kBatchThreads < c1 ? q + u * kBatchThreads : c1 - 1;
-              j[u] = stream_load(ic + e);
-              v[u] = stream_load(iv + e);
-            }
-#pragma unroll
-            for (int u = 0; u < kStreamAhead; ++u) xv[u] = ix[j[u]];
-#pragma unroll
-            for (int u = 0; u < kStreamAhead; ++u)
-              if (q + u * kBatchThreads < c1) s_prod[q + u * kBatchThreads - c0] = v[u] * xv[u];
-          }
+          if (c1 - c0 <= 2 * kBatchThreads)
+            stream_products<2>(ic, iv, ix, c0, c1, s_prod);
+          else if (c1 - c0 <= 4 * kBatchThreads)
+            stream_products<4>(ic, iv, ix, c0, c1, s_prod);
+          else
+            stream_products<kStreamAhead>(ic, iv, ix, c0, c1, s_prod);
           __syncthreads();
           const int32_t a = q0 > c0 ? q0 : c0, b = q1 < c1 ? q1 : c1;
           for (int32_t q = a; q < b; ++q) acc += s_prod[q - c0];

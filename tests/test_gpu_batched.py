@@ -146,3 +146,67 @@ def test_batch_fewer_instances_than_queues(ninst):
         torch.cuda.synchronize()
         check_spmv(w, range(w.ninst))
         del b
+
+
+class _Rows:
+    """A batch's workload: instances of n rows and n columns with the given row
+    lengths, random columns."""
+
+    def __init__(self, lengths, n, width, seed):
+        rng = np.random.default_rng(seed)
+        self.ninst, self.width = len(lengths), width
+        self.m = np.array([len(c) for c in lengths])
+        self.n = self.m
+        self.nnz = np.array([sum(c) for c in lengths])
+        assert all(len(c) == n for c in lengths)
+        pos, crd = [], []
+        for c in lengths:
+            pos.append(np.concatenate([[0], np.cumsum(c)]))
+            crd += [np.sort(rng.choice(n, k, replace=False)) for k in c]
+        self.host = [(p, np.concatenate(crd[i * n:(i + 1) * n])) for i, p in enumerate(pos)]
+        self.host_vals = rng.uniform(-1, 1, int(self.nnz.sum())).astype(np.float32)
+        self.host_x = rng.uniform(-1, 1, (self.ninst, n, width)).astype(np.float32)
+        self.pos = torch.tensor(np.concatenate(pos), dtype=torch.int32, device="cuda")
+        self.crd = torch.tensor(np.concatenate(crd), dtype=torch.int32, device="cuda")
+        self.vals = torch.tensor(self.host_vals, device="cuda")
+        self.x = self.B = torch.tensor(self.host_x, device="cuda").reshape(-1)
+        self.y = self.C = torch.full_like(self.x, float("nan"))
+
+    def expect(self):
+        """The products and, per row, the sum of their magnitudes, in 64 bits."""
+        out = np.zeros(self.host_x.shape)
+        size = np.zeros(self.host_x.shape)
+        e = 0
+        for i, (pos, crd) in enumerate(self.host):
+            rows = np.repeat(np.arange(len(pos) - 1), np.diff(pos))
+            v = self.host_vals[e:e + len(crd)].astype(np.float64)[:, None]
+            with np.errstate(invalid="ignore"):
+                p = v * self.host_x[i].astype(np.float64)[crd]
+            np.add.at(out[i], rows, p)
+            np.add.at(size[i], rows, np.abs(p))
+            e += len(crd)
+        return out, size
+
+
+def _run(w, op, lanes):
+    b = BT.Batch(w, op, lanes, rows_per_task=256)
+    b.capture()
+    for _ in range(3):
+        w.y.fill_(float("nan"))
+        b.launch_graph()
+        torch.cuda.synchronize()
+        out, size = w.expect()
+        got = w.y.cpu().numpy().astype(np.float64).reshape(out.shape)
+        # f32 sums of at most 65 products, each rounding at most 65 times.
+        assert np.all(np.abs(got - out) <= 65 * 2.0 ** -24 * size + 1e-30)
+
+
+# Rows of 1, 2, 3 and 4 entries make passes of 256, 512, 768 and 1024
+# entries, one more or less moves a pass over the edge of two, four or eight
+# entries in flight; 256 rows a task.
+@pytest.mark.parametrize("lanes", [0, 8])
+@pytest.mark.parametrize("length", [1, 2, 3, 4, 5, 16])
+def test_short_rows_spmv(length, lanes):
+    c = [[length] * 300, [length] * 255 + [length + 1] + [length] * 44,
+         [max(length - 1, 0)] + [length] * 299]
+    _run(_Rows(c, 300, 1, 5), 0, np.full(3, lanes, np.int32))
