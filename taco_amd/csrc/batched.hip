@@ -186,7 +186,13 @@ __global__ __launch_bounds__(kBatchThreads) void k_batch_spmv(
   });
 }
 
-__global__ __launch_bounds__(kBatchThreads) void k_batch_spmm(
+// WAVES: waves a SIMD that the registers leave room for.  The block of eight B
+// rows (K == 4 * lanes) would rather have 67 registers, 7 waves, than 64 (128
+// instances, 4.8 M rows, K = 32: 1532 us, 1564 with 8 waves); the other
+// widths need all 8 (K = 48 with 16 lanes, 2.6 M rows: 7945 us, 8696 with 7),
+// so a batch with an instance of another width takes those.
+template <int WAVES>
+__global__ __launch_bounds__(kBatchThreads, WAVES) void k_batch_spmm(
     Queues qs, int32_t K, const Task* __restrict__ tasks,
     const Inst* __restrict__ insts, const int32_t* __restrict__ pos,
     const int32_t* __restrict__ crd, const float* __restrict__ vals,
@@ -210,8 +216,9 @@ __global__ __launch_bounds__(kBatchThreads) void k_batch_spmm(
       // each, and pass them round, so that an entry costs the L1 little more
       // than its B row.  (Every lane loading every entry itself, three loads
       // an entry, kept the L1's data path as busy with entries as with B:
-      // 128 instances, 4.8 M rows, K = 32: 2243 -> 1730 us; and eight entries
-      // of every lane's own at a time, repeated past a row's end, 2750 us.)
+      // 128 instances, 4.8 M rows, K = 32: 2066 -> 1576 us; eight entries
+      // of every lane's own at a time, repeated past a row's end, took 1.2 times
+      // the first.)
       typedef float f32x4 __attribute__((ext_vector_type(4)));
       constexpr int kBRows = 8;
       const int turn = lane & (kBRows - 1);
@@ -224,29 +231,25 @@ __global__ __launch_bounds__(kBatchThreads) void k_batch_spmm(
           const float al = stream_load(iv + e);
           const int32_t jl = stream_load(ic + e);
           const int32_t left = end - q;
+          f32x4 b[kBRows];
           if (left >= kBRows) {
-            f32x4 b[kBRows];
-            float a[kBRows];
 #pragma unroll
-            for (int u = 0; u < kBRows; ++u) {
-              a[u] = __shfl(al, u, kBRows);
+            for (int u = 0; u < kBRows; ++u)
               b[u] = *(const f32x4*)(iB + (int64_t)__shfl(jl, u, kBRows) * K + 4 * lane);
-            }
 #pragma unroll
-            for (int u = 0; u < kBRows; ++u) acc += a[u] * b[u];
+            for (int u = 0; u < kBRows; ++u) acc += __shfl(al, u, kBRows) * b[u];
           } else {
-            f32x4 b[kBRows];
-            float a[kBRows];
 #pragma unroll
             for (int u = 0; u < kBRows; ++u) {
-              a[u] = __shfl(al, u, kBRows);
               const int32_t j = __shfl(jl, u, kBRows);
               if (u < left) b[u] = *(const f32x4*)(iB + (int64_t)j * K + 4 * lane);
               else b[u] = (f32x4){0.f, 0.f, 0.f, 0.f};
             }
 #pragma unroll
-            for (int u = 0; u < kBRows; ++u)
-              if (u < left) acc += a[u] * b[u];
+            for (int u = 0; u < kBRows; ++u) {
+              const float a = __shfl(al, u, kBRows);
+              if (u < left) acc += a * b[u];
+            }
           }
           q += kBRows;
         }
@@ -314,6 +317,7 @@ struct taco_hip_batch {
   const float* in = nullptr;  // x or B
   float* out = nullptr;       // y or C
   int grid = 0;
+  bool four_columns = false;  // note_columns
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   std::vector<Inst> host_insts;
@@ -331,6 +335,13 @@ void batch_free(taco_hip_batch* b) {
   delete b;
 }
 
+// Whether every instance's rows of C are 4 columns a lane.
+void note_columns(taco_hip_batch* b) {
+  b->four_columns = true;
+  for (const Inst& in : b->host_insts)
+    if (b->K != 4 * in.sched) b->four_columns = false;
+}
+
 // whole: every task through the per-XCD queues; otherwise tasks [t0, t0+nt)
 // through one queue.
 int launch_batch(taco_hip_batch* b, hipStream_t st, int32_t t0, int32_t nt, bool whole) {
@@ -343,8 +354,9 @@ int launch_batch(taco_hip_batch* b, hipStream_t st, int32_t t0, int32_t nt, bool
     hipLaunchKernelGGL(k_batch_spmv, dim3(grid), dim3(kBatchThreads), 0, st, qs, b->tasks,
                        b->insts, b->pos, b->crd, b->vals, b->in, b->out);
   else
-    hipLaunchKernelGGL(k_batch_spmm, dim3(grid), dim3(kBatchThreads), 0, st, qs, b->K,
-                       b->tasks, b->insts, b->pos, b->crd, b->vals, b->in, b->out);
+    hipLaunchKernelGGL(b->four_columns ? k_batch_spmm<7> : k_batch_spmm<8>, dim3(grid),
+                       dim3(kBatchThreads), 0, st, qs, b->K, b->tasks, b->insts, b->pos, b->crd,
+                       b->vals, b->in, b->out);
   TH_LAUNCH_CHECK("batched kernel");
   return 0;
 }
@@ -474,6 +486,7 @@ int taco_hip_batch_create(int32_t op, int32_t ninst, const int32_t* m,
   if (hipGetDevice(&dev) == hipSuccess)
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
   b->grid = cus * 8;
+  note_columns(b);
   *result = b;
   return 0;
 }
@@ -487,6 +500,7 @@ int taco_hip_batch_set_schedules(taco_hip_batch* b, const int32_t* sched) {
                "batch: instance %d has schedule %d, not a valid lane count", i, s);
     b->host_insts[(size_t)i].sched = s;
   }
+  note_columns(b);
   if (b->ninst > 0)
     TH_CHECK(hipMemcpyAsync(b->insts, b->host_insts.data(), sizeof(Inst) * b->ninst,
                             hipMemcpyHostToDevice, current_stream()));

@@ -210,3 +210,52 @@ def test_short_rows_spmv(length, lanes):
     c = [[length] * 300, [length] * 255 + [length + 1] + [length] * 44,
          [max(length - 1, 0)] + [length] * 299]
     _run(_Rows(c, 300, 1, 5), 0, np.full(3, lanes, np.int32))
+
+
+# Rows around the eight B rows that a team of lanes has in flight, at widths
+# of four columns a lane and others, alone and in one batch.
+@pytest.mark.parametrize("width,lanes", [(32, 8), (64, 16), (128, 32), (256, 64), (16, 8), (20, 8),
+                                         (48, 16), (33, 16), (100, 32)])
+def test_rows_around_a_block_spmm(width, lanes):
+    rng = np.random.default_rng(width)
+    c = [rng.choice([0, 1, 2, 7, 8, 9, 15, 16, 17, 64, 65], 120).tolist() for _ in range(3)]
+    _run(_Rows(c, 120, width, 6), 1, np.full(3, lanes, np.int32))
+    if 8 * lanes <= 256 and width == 4 * lanes:
+        _run(_Rows(c, 120, width, 7), 1, np.array([lanes, 2 * lanes, lanes], np.int32))
+
+
+@pytest.mark.parametrize("width,lanes", [(32, 8), (20, 8)])
+def test_spmm_schedules_replaced_after_capture(width, lanes):
+    """A captured launch stays right when the lane counts change."""
+    c = [[5] * 64, [9] * 64]
+    w = _Rows(c, 64, width, 8)
+    b = BT.Batch(w, 1, np.full(2, lanes, np.int32))
+    b.capture()
+    for again in (16, 8, 32):
+        b.set_schedules(np.array([lanes, again], np.int32))
+        w.y.fill_(float("nan"))
+        b.launch_graph()
+        torch.cuda.synchronize()
+        out, size = w.expect()
+        got = w.y.cpu().numpy().astype(np.float64).reshape(out.shape)
+        assert np.all(np.abs(got - out) <= 65 * 2.0 ** -24 * size)
+
+
+@pytest.mark.parametrize("op,width,lanes", [(0, 1, 0), (0, 1, 8), (1, 32, 8), (1, 20, 8)])
+def test_infinities_stay_in_their_rows(op, width, lanes):
+    """x values and B rows of infinities and NaN reach only the rows that name
+    them, also where a block is filled up past a row's end."""
+    c = [[3, 8, 1, 11, 0, 7, 9, 2] * 20] * 2
+    w = _Rows(c, 160, width, 9)
+    w.host_x[:, 5] = np.inf
+    w.host_x[:, 77] = np.nan
+    w.x.copy_(torch.tensor(w.host_x).reshape(-1))
+    b = BT.Batch(w, op, np.full(2, lanes, np.int32))
+    b.run()
+    torch.cuda.synchronize()
+    got = w.y.cpu().numpy().reshape(w.host_x.shape)
+    for i, (pos, crd) in enumerate(w.host):
+        rows = np.repeat(np.arange(160), np.diff(pos))
+        hit = np.unique(rows[np.isin(crd, [5, 77])])
+        clean = np.setdiff1d(np.arange(160), hit)
+        assert hit.size and np.isfinite(got[i][clean]).all() and not np.isfinite(got[i][hit]).any()
