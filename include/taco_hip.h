@@ -140,7 +140,12 @@ typedef struct taco_hip_schedule {
   int32_t algo;             /* taco_hip_algo */
   int32_t block_size;       /* threads per workgroup, multiple of 64 */
   int32_t items_per_thread; /* entries (NNZ_SPLIT) or merge items (MERGE_PATH) */
-  int32_t group_size;       /* lanes per row (GROUP_PER_ROW), power of 2 <= 64 */
+  int32_t group_size;       /* lanes per row (GROUP_PER_ROW), power of 2 <= 64.
+                               SpMM: lanes of a team, 8 .. 64, of at most 4
+                               columns each.  MERGE_PATH works by the wave
+                               whatever the team; items_per_thread below 256
+                               are those of one of its 64 / group_size teams,
+                               up to 256 a wave */
   int32_t rows_per_group;   /* rows per lane group (GROUP_PER_ROW) */
   int32_t reserved[3];
 } taco_hip_schedule;

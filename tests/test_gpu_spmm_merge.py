@@ -6,7 +6,7 @@ import pytest
 import torch
 
 import oracle
-from taco_amd import _lib
+from taco_amd import _lib, descriptors as D
 from taco_amd import workloads as W
 from tests import gpu_util as G
 
@@ -56,6 +56,41 @@ def test_infinities_stay_in_their_rows(K):
 def test_no_entries(K):
     A = W.Csr(300, 0, np.zeros(301, np.int32), np.zeros(0, np.int32), np.zeros(0))
     assert not G.spmm(A, np.zeros((0, K))).any()
+
+
+@pytest.mark.parametrize("group", [8, 16, 32, 64])
+@pytest.mark.parametrize("items", [1, 3, 16, 31, 64, 255])
+def test_items_of_small_teams(items, group):
+    """Items a wave takes for teams of every size, below the default of 256."""
+    A = _matrix()
+    B = W.uniform(A.n * 6, 10, W.STREAM_B).reshape(A.n, 6)
+    C = G.spmm(A, B, G.sched(_lib.MERGE_PATH, 256, items=items, group=group))
+    Ce, cond = oracle.exact_spmm(A, B)
+    rep = oracle.error_report(C, Ce, cond, TOL["f64"])
+    assert rep["ok"], rep
+
+
+def test_few_items_keep_their_pace():
+    """16 items a team of 8 lanes take at most twice as long as the default
+    (1.1 times; 3.3 times where a wave took the 16 items of one team)."""
+    m, K = 200_000, 4
+    A = W.csr_fixed(m, m, 16, 11)
+    a = G.csr_desc(A)
+    x, c = D.dense(torch.rand(m, K, dtype=torch.float64, device="cuda")), D.dense(
+        torch.empty(m, K, dtype=torch.float64, device="cuda"))
+    took = []
+    for s in (None, G.sched(_lib.MERGE_PATH, 256, items=16, group=8)):
+        best = []
+        for _ in range(5):
+            t0, t1 = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            t0.record()
+            for _ in range(10):
+                _lib.check(_lib.lib().taco_hip_spmm_compute(c.ptr, a.ptr, x.ptr, s))
+            t1.record()
+            torch.cuda.synchronize()
+            best.append(t0.elapsed_time(t1))
+        took.append(min(best))
+    assert took[1] < 2 * took[0], took
 
 
 def test_same_result_every_time():
