@@ -236,7 +236,12 @@ __global__ __launch_bounds__(256) void k_spmm_merge(
   typedef typename Adjacent<TC, CPL>::vec Out;
   const int lane = threadIdx.x % kWave;
   const int L = (K + CPL - 1) / CPL;
-  const int S = ONE ? 1 : kWave / L < kWave / U ? kWave / L : kWave / U;
+  // 4 groups for 10 to 16 lanes, though 10 to 12 leave room for 5 or 6: the
+  // sums of a row take fewer moves, and a chunk is a whole 64 entries.
+  const int S = ONE                 ? 1
+                : L > 9 && L <= 16  ? 4
+                : kWave / L < kWave / U ? kWave / L
+                                    : kWave / U;
   const int chunk = kWave / (S * U) * (S * U);
   const int sub = ONE ? 0 : lane / L, kl = ONE ? lane : lane % L;
   const bool owns = sub < S && kl < L;  // lanes left over repeat others' loads
@@ -477,11 +482,14 @@ __global__ __launch_bounds__(kFixupWaves * kWave) void k_spmm_merge_fixup(
 }
 
 // Adjacent columns a lane of the merge kernel owns: 16 bytes of f32 or f64
-// (one column below that width), except f64 rows of 33 to 64 columns, where
-// a wave to a B row is faster (1M-row power-law matrix, K = 64: 1210 us
-// against 1245 with two columns a lane).  Wider f64 rows take strided
-// columns (kStrided: 326,797 uniform rows of 30, K = 102: 1272 us against
-// 1307 with adjacent ones; 200,000 banded rows, K = 128: 406 against 430).
+// (one column below that width), except f64 rows of 33 to 64 columns, which
+// take a wave to a B row.  Two columns a lane, two or three B rows to a load,
+// are no better throughout (one : two columns, f64): 300,000 power-law rows
+// of 16, K = 33 287 : 305 us, 48 298 : 304, 64 392 : 401; 300,000 banded rows
+// of 20 231 : 198, 259 : 241, 346 : 339; 100,000 uniform rows of 16 100 : 98,
+// 105 : 104, 136 : 138.  Wider f64 rows take strided columns (kStrided:
+// 326,797 uniform rows of 30, K = 102: 1272 us against 1307 with adjacent
+// ones; 200,000 banded rows, K = 128: 406 against 430).
 template <typename TC>
 int merge_cols(int32_t K) {
   const int wide = 16 / (int)sizeof(TC);
@@ -560,15 +568,21 @@ int run_spmm(const CsrView& a, int32_t K, const TA* B, TC* C,
     // (200,000 uniform rows of 16, f64: 219 us, now 71; 32 items 127, now 67;
     // 256 items 67).
     if (ipt < 256) ipt = ipt * (kWave / G) < 256 ? ipt * (kWave / G) : 256;
+    const int cols = merge_cols<TC>(K);
+    const bool one = (K + cols - 1) / cols > 32;
     const int64_t total = (int64_t)a.m + a.nnz;
+    // f64 rows of 17 to 32 columns in fewer waves than are resident (8192):
+    // 192 items each, f64, K = 24, 192 against 256: 100,000 uniform rows of
+    // 16 67.9 : 76.6 us, 100,000 banded of 20 58.1 : 61.7; in more waves than
+    // that, 150,000 uniform rows, 104.6 : 100.9.  (f32 rows of 16 columns
+    // 41.7 : 37.5.)
+    if (sizeof(TC) == 8 && K > 16 && !one && ipt > 192 && total < (int64_t)ipt * 8192) ipt = 192;
     const int64_t nteams = (total + ipt - 1) / ipt;
     const size_t row_bytes = ((size_t)nteams * sizeof(int32_t) + 255) / 256 * 256;
     void* ws = workspace(row_bytes + (size_t)nteams * K * sizeof(TC), 1);
     if (!ws) return 1;
     int32_t* crow = (int32_t*)ws;
     TC* cval = (TC*)((char*)ws + row_bytes);
-    const int cols = merge_cols<TC>(K);
-    const bool one = (K + cols - 1) / cols > 32;
     unsigned grid = (unsigned)((nteams * kWave + bs - 1) / bs);
     // Narrow rows: 16 groups of 4 lanes, 4 steps each.
     const int steps = (K + cols - 1) / cols <= 4 ? 4 : 8;
