@@ -25,38 +25,67 @@ def _csr(rows, n, seed):
     return W.Csr(len(rows), n, pos, crd, vals)
 
 
-def _pick(rng, lo, span, count):
-    """count distinct sorted columns of [lo, lo + span), both ends among them."""
-    inner = rng.choice(span - 2, count - 2, replace=False) + 1 if count > 2 else []
-    return lo + np.sort(np.concatenate([[0], inner, [span - 1]])).astype(np.int64)
-
-
-def _case(span, la, lb, seed, reverse=False):
-    """C rows of la * lb candidates whose columns span exactly `span`; 37
-    rows of C, every B row of a C row from the same window."""
+def _case(span, la, lb, distinct, seed, reverse=False):
+    """C rows of la * lb candidates of exactly `distinct` columns, which span
+    exactly `span`; 37 rows of C.  Every column is dealt to one of the row's
+    la B rows, which are then filled up to lb with others."""
     rng = np.random.default_rng(seed)
     m, n = 37, span + 4096
     brows, arows = [], []
     for i in range(m):
         lo = int(rng.integers(0, n - span + 1))
+        cols = np.concatenate([[0], rng.choice(span - 2, distinct - 2, replace=False) + 1, [span - 1]])
+        cols = rng.permutation(lo + cols)
         arows.append(range(i * la, (i + 1) * la))
-        for _ in range(la):
-            r = _pick(rng, lo, span, min(lb, span))
+        for q in range(la):
+            own = cols[q::la]
+            assert len(own) <= lb
+            more = rng.choice(np.setdiff1d(cols, own), lb - len(own), replace=False)
+            r = np.sort(np.concatenate([own, more])).astype(np.int64)
             brows.append(r[::-1] if reverse else r)
     return _csr(arows, m * la, seed), _csr(brows, n, seed + 1)
 
 
+def _shape_of(A, B, i):
+    """Row i of C: its candidates, its distinct columns and their span."""
+    cols = np.concatenate([B.crd[B.pos[j]:B.pos[j + 1]] for j in A.crd[A.pos[i]:A.pos[i + 1]]])
+    return len(cols), len(np.unique(cols)), int(cols.max()) - int(cols.min()) + 1
+
+
 CASES = [
-    # span, A entries, B entries a row
-    ("flags_small", (65, 3, 64)), ("flags_edge", (1024, 5, 70)), ("bits_edge", (1025, 5, 70)),
-    ("bits_mid", (20000, 9, 33)), ("bits_top", (32768, 12, 40)), ("sort_2", (32769, 2, 64)),
-    ("sort_2_65", (40000, 13, 5)), ("sort_4", (40000, 3, 43)), ("sort_4_top", (40000, 4, 64)),
-    ("sort_8", (70000, 257, 1)), ("sort_8_top", (70000, 4, 128)), ("sort_16", (70000, 9, 57)),
-    ("sort_16_top", (70000, 8, 128)), ("hash", (70000, 41, 25)),
-    # distinct columns around the staged-search limit (682) and the slots (1024)
-    ("staged_top", (60000, 11, 62)), ("unstaged", (60000, 11, 63)), ("slots", (50000, 8, 128)),
-    ("over_slots", (300000, 30, 60)), ("long_b", (900, 3, 700)), ("many_a", (1000, 200, 3)),
+    # span, A entries, entries of a B row, distinct columns
+    ("flags_small", (65, 3, 64, 65)), ("flags_edge", (1024, 5, 70, 300)),
+    ("flags_full", (1024, 16, 64, 1024)), ("bits_edge", (1025, 5, 70, 300)),
+    ("bits_mid", (20000, 9, 33, 250)), ("bits_top", (32768, 12, 40, 400)),
+    ("sort_2_65", (40000, 13, 5, 60)), ("sort_2", (32769, 2, 64, 128)),
+    ("sort_4", (40000, 3, 43, 120)), ("sort_4_top", (40000, 4, 64, 256)),
+    ("sort_8", (70000, 257, 1, 257)), ("sort_8_top", (70000, 4, 128, 500)),
+    ("sort_16", (70000, 9, 57, 513)), ("sort_16_top", (70000, 8, 128, 1000)),
+    ("hash", (70000, 41, 25, 900)), ("hash_full", (70000, 11, 100, 1024)),
+    # distinct columns around the staged search (682) and the sums in LDS (1024)
+    ("staged_top", (60000, 11, 62, 682)), ("unstaged", (60000, 11, 63, 683)),
+    ("slots", (50000, 8, 128, 1024)), ("over_slots", (50000, 41, 25, 1025)),
+    ("staged_top_bits", (20000, 11, 62, 682)), ("unstaged_bits", (20000, 11, 63, 683)),
+    ("over_slots_bits", (20000, 41, 25, 1025)),
+    ("far_over_slots", (300000, 30, 60, 1700)), ("long_b", (900, 3, 700, 800)),
+    ("many_a", (1000, 200, 3, 400)),
 ]
+
+
+def test_cases_are_what_they_are_called():
+    """Candidates, columns and spans of the cases, counted on the host."""
+    for name, (span, la, lb, distinct) in CASES:
+        A, B = _case(span, la, lb, distinct, seed=len(name) * 31 + span)
+        for i in (0, 17, 36):
+            assert _shape_of(A, B, i) == (la * lb, distinct, span), name
+        route = ("flags" if span <= 1024 else "bits" if span <= 32768 else
+                 "sort" if la * lb <= 1024 else "hash")
+        kind = name.split("_")[0]
+        if kind in ("flags", "bits", "sort", "hash"):
+            assert kind == route, name
+        if kind == "sort":
+            values = int(name.split("_")[1])  # a lane: at most 64 times as many candidates
+            assert max(32 * values, 64) < la * lb <= 64 * values, name
 
 
 @pytest.mark.parametrize("name,shape", CASES, ids=[c[0] for c in CASES])
@@ -155,3 +184,30 @@ def test_heavy_rows_together_keep_their_pace():
         for p in (c.level_ptr(1, 0), c.level_ptr(1, 1), c.vals_ptr()):
             L.taco_hip_unified_free(ctypes.c_void_p(p))
     assert took["together"] < 3 * took["spread"], took
+
+
+@pytest.mark.parametrize("ends,outside", [((10, 900), 5000), ((10, 900), 2), ((10, 30000), 60000),
+                                          ((10, 30000), 2)],
+                         ids=["flags_above", "flags_below", "bits_above", "bits_below"])
+@pytest.mark.parametrize("long", [False, True], ids=["hash", "over_hash"])
+def test_columns_outside_the_ends(ends, outside, long):
+    """B rows that are not sorted inside and hold columns beyond their first
+    and last ones: noticed while the columns are collected, and the row is
+    done again by the hash set (of up to 1024 columns) or the global sort."""
+    rng = np.random.default_rng(outside)
+    m, la = 11, 40
+    lb = 40 if long else 20
+    brows, arows = [], []
+    for i in range(m):
+        arows.append(range(i * la, (i + 1) * la))
+        for q in range(la):
+            inner = rng.choice(np.arange(ends[0] + 1, ends[1]), lb - 2, replace=False)
+            if (i + q) % 3 == 0:
+                inner[rng.integers(0, lb - 2)] = outside
+            brows.append(np.concatenate([[ends[0]], rng.permutation(inner), [ends[1]]]))
+    A, B = _csr(arows, m * la, 5), _csr(brows, 70000, 6)
+    if long:
+        assert ends[1] < 1024 or _shape_of(A, B, 0)[1] > 1024
+    else:
+        assert _shape_of(A, B, 0)[1] <= 1024
+    _check(A, B)
