@@ -579,10 +579,8 @@ int run_spmv(const CsrView& a, const T* x, T* y, const taco_hip_schedule& s,
     k_spmv_merge<T, K><<<(unsigned)nblocks, 256, 0, st>>>(                 \
         a.m, a.nnz, a.pos, a.crd, (const T*)a.vals, x, y, crow, cval);     \
     break;
-    switch (k) {
+    switch (k) {  // one of these, as required above
       TH_MP(2) TH_MP(4) TH_MP(6) TH_MP(8) TH_MP(12) TH_MP(16)
-      default:
-        return fail("spmv: items_per_thread %d unsupported for MERGE_PATH", k);
     }
 #undef TH_MP
     TH_LAUNCH_CHECK("k_spmv_merge");
