@@ -25,12 +25,15 @@ __device__ __forceinline__ T stream_load(const T* p) {
 // one gather each instead of 21 dependent loads.  Up to kGuessRows rows the
 // first round instead tests 16 pivots around the row that equal rows would
 // put at d, at distances of 16 rows and four times more each: where rows are
-// alike, one more round finishes (100,000 rows of 10: SpMV tiles 14.3 -> 11.5
-// us; SpMM, 400,009 banded rows: 179 -> 170).  On larger matrices the guess
-// of a power-law matrix is thousands of rows off, and its pivots are every
-// tile's own where the evenly spaced ones are all tiles' (2M rows, f32 SpMV:
-// 304 us, 319 with the guess; 1M rows, f64 SpMM: 1210 and 1237).  Every lane
-// returns r.
+// alike, one more round finishes.  Whole calls with the guess and without:
+// SpMV, f64, uniform, 100,000 rows of 10 15.2 : 15.4 us, 500,000 of 16 68.6 :
+// 70.8; f32, 500,000 banded rows of 16 23.8 : 25.9; SpMM, f32, 400,009 banded
+// rows, K = 33 175 : 181.  A power-law matrix pays for a round that finds
+// little: f64, 100,000 rows of 10 13.2 : 12.7, 200,000 of 16 27.9 : 27.3,
+// 500,000 65.5 : 65.1.  On larger ones the guess is thousands of rows off, and
+// its pivots are every tile's own where the evenly spaced ones are all tiles'
+// (2M rows, f32, the tiles alone: 319 : 304 us; 1M rows, f64 SpMM: 1237 :
+// 1210).  Every lane returns r.
 constexpr int64_t kGuessRows = 1 << 19;
 __device__ __forceinline__ int64_t wave_merge_search(const int32_t* pos,
                                                      int64_t m, int64_t nnz,

@@ -57,10 +57,11 @@ PLAN_CLASS = SPMV_NAMES.index("slab_plan")
 
 
 # bf16 SpMM goes to the MFMA kernel by rule: the network's classes were
-# timed in f64 and f32, the MFMA kernel exists only for bf16 (K a multiple of
-# 4), and it is the fastest bf16 form measured (0.89 ms on the 2M-row
-# power-law matrix at K = 64, against 2.06 ms for the merge class the
-# network picks there).  Its index lies past the network's classes.
+# timed in f64 and f32, and the MFMA kernel exists only for bf16 (K a multiple
+# of 4).  The rule dates from when it took 0.89 ms on the 2M-row power-law
+# matrix at K = 64 and the merge class 2.06; the merge path now takes 0.84
+# there (MFMA 0.83), 107 us on 200,000 power-law rows (MFMA 127) and 84 on
+# 200,000 banded ones (MFMA 74).  Its index lies past the network's classes.
 RULE_MFMA = N_CLASSES
 
 
