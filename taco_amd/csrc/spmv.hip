@@ -286,21 +286,25 @@ __global__ __launch_bounds__(256) void k_spmv_merge_fixup(
   if (first >= nblocks) return;
   const int32_t r = b < nblocks ? carry_row[b] : -1;
   T s = b < nblocks ? carry_val[b] : T(0);
-  // The row before the wave's first slot.
+  // The rows before the wave's first slot and after its last.
   const int32_t outside = first > 0 ? carry_row[first - 1] : -1;
+  const int32_t after = first + kWave < nblocks ? carry_row[first + kWave] : -1;
   int32_t before = __shfl_up(r, 1, kWave);
   if (lane == 0) before = outside;
   const bool head = r >= 0 && r < m && before != r;
   const T old = head ? y[r] : T(0);
-  // s: the sum of the lane's run from the lane on.
+  // s: the sum of the lane's run from the lane on.  Most waves hold none of
+  // two slots.
+  if (__ballot(r >= 0 && lane > 0 && before == r)) {
 #pragma unroll
-  for (int off = 1; off < kWave; off <<= 1) {
-    const T u = __shfl_down(s, off, kWave);
-    const int32_t ru = __shfl_down(r, off, kWave);
-    if (lane + off < kWave && ru == r) s += u;
+    for (int off = 1; off < kWave; off <<= 1) {
+      const T u = __shfl_down(s, off, kWave);
+      const int32_t ru = __shfl_down(r, off, kWave);
+      if (lane + off < kWave && ru == r) s += u;
+    }
   }
   const int32_t last = __builtin_amdgcn_readlane(r, kWave - 1);
-  const bool open = head && r == last;
+  const bool open = head && r == last && after == last;
   if (__ballot(open)) {
     T more = 0;
     for (int32_t c = first + kWave + lane;; c += kWave) {
