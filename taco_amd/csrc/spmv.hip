@@ -338,7 +338,8 @@ __global__ __launch_bounds__(256) void k_spmv_merge_fixup(
 // would take 25 for nine neighbouring rows of 5000 and not 8.4).  The number of
 // workgroups is odd, so that long rows at a power of two's distance are spread
 // as well; small grids are widened to kSmallSpread (1000 rows of 10 in 33
-// workgroups 2.4 us of kernel time, in 5 3.5).
+// workgroups 2.4 us of kernel time, in 5 3.5).  `stride` is the grid's size: a
+// kernel that reads gridDim needs arguments from the runtime, 0.3 us a launch.
 constexpr int kSmallOwn = 16;
 constexpr int kSmallThreads = 1024;
 constexpr int kSmallAhead = 16;
@@ -385,8 +386,9 @@ __device__ __forceinline__ T small_row_sum(int32_t q0, int32_t q1, int lane,
 
 template <typename T, int G>
 __global__ __launch_bounds__(kSmallThreads) void k_spmv_small(
-    int32_t m, const int32_t* __restrict__ pos, const int32_t* __restrict__ crd,
-    const T* __restrict__ vals, const T* __restrict__ x, T* __restrict__ y) {
+    int32_t m, int32_t stride, const int32_t* __restrict__ pos,
+    const int32_t* __restrict__ crd, const T* __restrict__ vals, const T* __restrict__ x,
+    T* __restrict__ y) {
   constexpr int kRows = kSmallThreads / G;
   constexpr int kTeams = kSmallThreads / kSmallTeam, kWaves = kSmallThreads / kWave;
   constexpr int kAhead = 4;
@@ -394,8 +396,8 @@ __global__ __launch_bounds__(kSmallThreads) void k_spmv_small(
   __shared__ T s_sum[kWaves];
   __shared__ int s_count[3];
   const int tid = threadIdx.x, sub = tid % G, slot = tid / G;
-  const int64_t row0 = blockIdx.x, stride = gridDim.x;
-  const int64_t i = row0 + slot * stride;
+  const int64_t row0 = blockIdx.x;
+  const int64_t i = row0 + (int64_t)slot * stride;
   const int32_t p0 = i < m ? pos[i] : 0, p1 = i < m ? pos[i + 1] : 0;
   const bool is_long = p1 - p0 > kSmallOwn * G;
   if (tid < 3) s_count[tid] = 0;
@@ -429,20 +431,20 @@ __global__ __launch_bounds__(kSmallThreads) void k_spmv_small(
   // Each long row's sum does not depend on the order of the lists.  Waves
   // take rows from the last wave on, teams from the first.
   for (int k = tid / kSmallTeam; k < s_count[0]; k += kTeams) {
-    const int64_t row = row0 + s_team[k] * stride;
+    const int64_t row = row0 + (int64_t)s_team[k] * stride;
     T s = small_row_sum<T, kSmallTeam>(pos[row], pos[row + 1], tid % kSmallTeam, crd, vals, x);
 #pragma unroll
     for (int off = kSmallTeam / 2; off > 0; off >>= 1) s += __shfl_xor(s, off, kSmallTeam);
     if (tid % kSmallTeam == 0) y[row] = s;
   }
   for (int k = kWaves - 1 - tid / kWave; k < s_count[1]; k += kWaves) {
-    const int64_t row = row0 + s_wave[k] * stride;
+    const int64_t row = row0 + (int64_t)s_wave[k] * stride;
     T s = small_row_sum<T, kWave>(pos[row], pos[row + 1], tid % kWave, crd, vals, x);
     s = wave_sum(s);
     if (tid % kWave == 0) y[row] = s;
   }
   for (int k = 0; k < s_count[2]; ++k) {
-    const int64_t row = row0 + s_all[k] * stride;
+    const int64_t row = row0 + (int64_t)s_all[k] * stride;
     T s = small_row_sum<T, kSmallThreads>(pos[row], pos[row + 1], tid, crd, vals, x);
     s = wave_sum(s);
     if (tid % kWave == 0) s_sum[tid / kWave] = s;
@@ -488,8 +490,8 @@ void launch_spmv_small(const CsrView& a, const T* x, T* y, hipStream_t st) {
   const unsigned grid = (unsigned)((need > spread ? need : spread) | 1);
 #define TH_SMALL(G)                                                            \
   case G:                                                                      \
-    k_spmv_small<T, G><<<grid, kSmallThreads, 0, st>>>(a.m, a.pos, a.crd,      \
-                                             (const T*)a.vals, x, y);          \
+    k_spmv_small<T, G><<<grid, kSmallThreads, 0, st>>>(                        \
+        a.m, (int32_t)grid, a.pos, a.crd, (const T*)a.vals, x, y);             \
     break;
   switch (g) {
     TH_SMALL(2) TH_SMALL(4) TH_SMALL(8) TH_SMALL(16) TH_SMALL(32) TH_SMALL(64)
