@@ -190,7 +190,9 @@ __global__ __launch_bounds__(kBatchThreads) void k_batch_spmv(
 // rows (K == 4 * lanes) would rather have 67 registers, 7 waves, than 64 (128
 // instances, 4.8 M rows, K = 32: 1532 us, 1564 with 8 waves); the other
 // widths need all 8 (K = 48 with 16 lanes, 2.6 M rows: 7945 us, 8696 with 7),
-// so a batch with an instance of another width takes those.
+// so a batch with an instance of another width takes those (90
+// instances of up to 60,000 rows, K = 20: 1685 us, 1748 with 7; though 20 of
+// up to 200,000, K = 16: 1369 and 1308).
 template <int WAVES>
 __global__ __launch_bounds__(kBatchThreads, WAVES) void k_batch_spmm(
     Queues qs, int32_t K, const Task* __restrict__ tasks,
@@ -231,24 +233,30 @@ __global__ __launch_bounds__(kBatchThreads, WAVES) void k_batch_spmm(
           const float al = stream_load(iv + e);
           const int32_t jl = stream_load(ic + e);
           const int32_t left = end - q;
+          // Values are passed round beside the columns where registers allow.
           f32x4 b[kBRows];
+          float a[kBRows];
+          const auto value = [&](int u) { return WAVES < 8 ? a[u] : __shfl(al, u, kBRows); };
           if (left >= kBRows) {
 #pragma unroll
-            for (int u = 0; u < kBRows; ++u)
+            for (int u = 0; u < kBRows; ++u) {
+              if (WAVES < 8) a[u] = __shfl(al, u, kBRows);
               b[u] = *(const f32x4*)(iB + (int64_t)__shfl(jl, u, kBRows) * K + 4 * lane);
+            }
 #pragma unroll
-            for (int u = 0; u < kBRows; ++u) acc += __shfl(al, u, kBRows) * b[u];
+            for (int u = 0; u < kBRows; ++u) acc += value(u) * b[u];
           } else {
 #pragma unroll
             for (int u = 0; u < kBRows; ++u) {
+              if (WAVES < 8) a[u] = __shfl(al, u, kBRows);
               const int32_t j = __shfl(jl, u, kBRows);
               if (u < left) b[u] = *(const f32x4*)(iB + (int64_t)j * K + 4 * lane);
               else b[u] = (f32x4){0.f, 0.f, 0.f, 0.f};
             }
 #pragma unroll
             for (int u = 0; u < kBRows; ++u) {
-              const float a = __shfl(al, u, kBRows);
-              if (u < left) acc += a * b[u];
+              const float v = value(u);
+              if (u < left) acc += v * b[u];
             }
           }
           q += kBRows;
